@@ -1,0 +1,104 @@
+"""g4a_gemm16 / g4a_gemm16_ws / g4a_gemm16_geglu at the edges of every output tile the launch
+plan can take (csrc/gemm.hip kTiles): ragged tokens and outputs, one k-stage, fewer stages than
+the pipeline holds, grouped matrices whose last tiles are partly empty, and a split with the
+smallest tile. Products against float64 (on the GPU, the operands being f16 exactly):
+
+    |got - f16(ref)| <= one f16 ulp of ref + K 2^-24 sum|a w|
+
+the f32 accumulation bound in any order, plus the f16 rounding of a value that far off. The
+gate/up form must equal g4a_gemm16 followed by g4a_geglu16, which divides, code for code.
+"""
+import numpy as np
+import pytest
+import torch
+
+import slang_amd as sa
+from slang_amd.decoder import geglu16
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def operands(M, K, ns, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    a = torch.randn(M, K, device=DEV, generator=g).half()
+    return a, [(0.05 * torch.randn(n, K, device=DEV, generator=g)).half() for n in ns]
+
+
+def close(got, a, w, what):
+    ref = a.double() @ w.double().T
+    mag = a.double().abs() @ w.double().abs().T
+    r16 = ref.half().double()
+    ulp = torch.clamp(2.0 ** (torch.floor(torch.log2(ref.abs().clamp_min(2.0 ** -14))) - 10), min=2.0 ** -24)
+    bad = (got.double() - r16).abs() > ulp + a.shape[1] * 2.0 ** -24 * mag
+    assert not bad.any(), f"{what}: {int(bad.sum())} of {bad.numel()} products off"
+
+
+# the tile that the plan takes, by its measured costs: 256 x 256, 256 x 192, 192 x 128,
+# 128 x 128, 64 x 128
+SHAPES = [(2047, 64, (24576,)), (2040, 192, (12288, 12160)), (1000, 128, (24448,)), (2047, 128, (4096, 512, 512)),
+          (1893, 192, (3072,)), (1893, 64, (2048, 384, 640)), (1024, 320, (2048, 512)), (513, 64, (4096,)),
+          (1, 64, (128,)), (65, 448, (384, 128)), (63, 128, (24576,))]
+
+
+@pytest.mark.parametrize("M,K,ns", SHAPES)
+def test_every_tile_matches_float64(M, K, ns):
+    print(f"gemm16 M {M} K {K} n {ns}", flush=True)
+    a, ws = operands(M, K, ns, M + K)
+    outs = [torch.full((M + 2, n), 7.0, device=DEV, dtype=torch.float16) for n in ns]
+    sa.gemm16(a, [(w, o[:M], None) for w, o in zip(ws, outs)])
+    for i, (w, o) in enumerate(zip(ws, outs)):
+        close(o[:M], a, w, f"matrix {i}")
+        assert (o[M:] == 7.0).all(), "stores past M"
+    # the q path: srq of the same f16 products, exactly
+    q = torch.full((M + 2, ns[0]), 7.0, device=DEV)
+    sa.gemm16(a, [(ws[0], q[:M], 0.03125)])
+    want = torch.clamp(torch.round(outs[0][:M].float() / 0.03125), -128, 127) * 0.03125
+    assert torch.equal(q[:M], want) and (q[M:] == 7.0).all()
+
+
+@pytest.mark.parametrize("M,K,ns", [(77, 4096, (128, 384)), (1, 8192, (128,)), (1000, 12288, (1536,)), (130, 6144, (1536,))])
+def test_split_tiles_match_float64_and_repeat(M, K, ns):
+    print(f"gemm16 split M {M} K {K} n {ns}", flush=True)
+    a, ws = operands(M, K, ns, M + K)
+    outs = [torch.full((M + 2, n), 7.0, device=DEV, dtype=torch.float16) for n in ns]
+    mats = [(w, o[:M], None) for w, o in zip(ws, outs)]
+    gws = sa.GemmWorkspace()
+    gws.get(sa.gemm16_ws_bytes(M, K, ns))
+    gws.buf[sa._lib.GEMM_TICKET_BYTES:].fill_(0xFF)  # stale partials are NaN and must not be read
+    sa.gemm16(a, mats, gws)
+    first = [o.clone() for o in outs]
+    sa.gemm16(a, mats, gws)
+    for i, (w, o, f) in enumerate(zip(ws, outs, first)):
+        assert torch.equal(o, f), "a repeat call differs"
+        close(o[:M], a, w, f"matrix {i}")
+        assert (o[M:] == 7.0).all(), "stores past M"
+    assert not gws.buf[:sa._lib.GEMM_TICKET_BYTES].any(), "tickets left non-zero"
+
+
+def gelu_table(step):
+    v = (np.arange(256) - 128).astype(np.float64) * step
+    return torch.from_numpy((0.5 * v * (1 + np.tanh(0.7978845608028654 * (v + 0.044715 * v ** 3)))).astype(np.float32)).to(DEV)
+
+
+def geglu_pair(a, wg, wu, gq, uq, oq, lut):
+    M, n = a.shape[0], wg.shape[0]
+    out = torch.full((M + 2, n), 7.0, device=DEV, dtype=torch.float16)
+    sa.gemm16_geglu(a, wg, wu, gq, uq, oq, out=out[:M], gelu_lut=lut)
+    g, u = (torch.empty(M, n, device=DEV, dtype=torch.float16) for _ in range(2))
+    for w, o in ((wg, g), (wu, u)):
+        pad = torch.zeros(-n % 128, a.shape[1], device=DEV, dtype=torch.float16)
+        full = torch.empty(M, n + len(pad), device=DEV, dtype=torch.float16)
+        sa.gemm16(a, [(torch.cat([w, pad]), full, None)])
+        o.copy_(full[:, :n])
+    assert (out[M:] == 7.0).all(), "stores past M"
+    return out[:M], geglu16(g, u, gq, uq, oq, gelu_lut=lut)
+
+
+@pytest.mark.parametrize("M,K,n", [(2047, 64, 12288), (1000, 128, 12224), (1893, 192, 1536), (1024, 320, 1216), (65, 64, 64)])
+@pytest.mark.parametrize("table", [True, False])
+def test_geglu_tiles_equal_the_divided_form(M, K, n, table):
+    print(f"gemm16_geglu M {M} K {K} n {n} table {table}", flush=True)
+    a, (wg, wu) = operands(M, K, (n, n), M + n)
+    got, want = geglu_pair(a, wg, wu, 0.013, 0.021, 0.0073, gelu_table(0.013) if table else None)
+    assert torch.equal(got, want), f"{int((got != want).sum())} codes differ"
