@@ -179,6 +179,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm16_kernel(Gemm16Args g
         }
     };
 
+    float lut_entry = 0.0f;  // out before the stages, used after them
+    if (GEGLU && g.lut && tid < 256) lut_entry = g.lut[tid];
     float16v acc[NB][MB];
 #pragma unroll
     for (int a = 0; a < NB; ++a)
@@ -312,8 +314,9 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm16_kernel(Gemm16Args g
     };
     if constexpr (GEGLU) {
         constexpr int SR = WO * 2 + 16;
-        static_assert(NW * 32 * SR <= ST * STB, "the staged rows fit the operand stages");
+        static_assert(NW * 32 * SR + 1024 <= ST * STB && 64 * NW >= 256, "the staged rows and the table fit the stages");
         char* sg = lds + wave * 32 * SR;
+        float* table = reinterpret_cast<float*>(lds + NW * 32 * SR);
         auto blocks = [&](auto&& code) {
 #pragma unroll
             for (int b = 0; b < MB; ++b) {
@@ -330,7 +333,19 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm16_kernel(Gemm16Args g
                 store_rows(Idx<2>{}, sg, b, g.out[0]);
             }
         };
-        blocks([&](float gv, float uv) { return geglu_code(gv, uv, g.gq, g.uq, g.oq, g.lut); });
+        if (g.lut && srq_fast(g.gq) && srq_fast(g.uq) && srq_fast(g.oq)) {
+            // geglu_code's arithmetic with srq_index for its three divisions and the GELU table in
+            // LDS: read from memory, each of a lane's lookups was a dependent 64-address gather
+            const SrqStep tg = srq_step(g.gq), tu = srq_step(g.uq), to = srq_step(g.oq);
+            if (tid < 256) table[tid] = lut_entry;
+            __syncthreads();
+            blocks([&](float gv, float uv) {
+                const float y = pin(table[(int)srq_index(gv, tg) + 128] * pin(srq_index(uv, tu) * tu.s));
+                return (half_t)srq_index(y, to);
+            });
+        } else {
+            blocks([&](float gv, float uv) { return geglu_code(gv, uv, g.gq, g.uq, g.oq, g.lut); });
+        }
         return;
     }
     const float oq = g.out_q[p], alpha = g.alpha[p];
@@ -353,7 +368,12 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm16_kernel(Gemm16Args g
                 store_rows(Idx<4>{}, sg, b, g.out[p]);
             }
         };
-        blocks([&](float x) { return srq(x, oq); });
+        if (srq_fast(oq)) {
+            const SrqStep t = srq_step(oq);
+            blocks([&](float x) { return srq_index(x, t) * oq; });
+        } else {
+            blocks([&](float x) { return srq(x, oq); });
+        }
         return;
     }
     constexpr int SR = WO * 2 + 16;

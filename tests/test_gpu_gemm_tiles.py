@@ -102,3 +102,20 @@ def test_geglu_tiles_equal_the_divided_form(M, K, n, table):
     a, (wg, wu) = operands(M, K, (n, n), M + n)
     got, want = geglu_pair(a, wg, wu, 0.013, 0.021, 0.0073, gelu_table(0.013) if table else None)
     assert torch.equal(got, want), f"{int((got != want).sum())} codes differ"
+
+
+@pytest.mark.parametrize("step", [0.02, 0.0137, 0.3330001, 1e-6, 1e-14, 1e14])
+@pytest.mark.parametrize("scale", [1.0, 2.0])
+def test_geglu_codes_of_every_f16_value(step, scale):
+    """Every finite f16 value as a gate and as an up product (scale 2: the largest overflow to
+    f16 infinities), at steps the epilogue quantises by refined products and, at the two last,
+    by division: the codes equal the divided form's."""
+    print(f"geglu every f16 step {step} scale {scale}", flush=True)
+    v = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    v = torch.where(torch.isfinite(v), v, torch.zeros(())).half().to(DEV)
+    a = (scale * torch.eye(64, device=DEV)).half()
+    wg, wu = v.view(1024, 64), v.view(1024, 64).flip(0).contiguous()
+    lut = gelu_table(0.02) + 0.25 * torch.sign(gelu_table(0.02))
+    for w1, w2, steps in ((wg, wu, (step, 0.02, 0.05)), (wu, wg, (0.02, step, 0.05)), (wg, wg, (0.02, 0.02, step))):
+        got, want = geglu_pair(a, w1, w2, *steps, lut)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), f"{int((got != want).sum())} codes differ"
