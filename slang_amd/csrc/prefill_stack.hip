@@ -87,76 +87,124 @@ __global__ __launch_bounds__(256) void rows_tail_kernel(TailArgs a) {
     }
 }
 
+// Calls body(over) with over(x) = x / r, correctly rounded, for r the same in every lane. For r in
+// [2^-40, 2^40] the quotient is x / r's product form refined twice by its exact residual, as
+// srq_index (common.hpp) does and for the same reason; otherwise (a row of zero or infinite
+// values, NaN) it divides. |x| <= r sqrt(n) here, so no step overflows; below |x| / r = 2^-100
+// the last bit may differ from the division's, far under what any use of it keeps.
+template <class F>
+__device__ __forceinline__ void with_quotient(float r, F&& body) {
+    if (r >= 0x1p-40f && r <= 0x1p40f) {
+        const float y = 1.0f / r;
+        body([&](float x) {
+            float q = x * y;
+            q = __builtin_fmaf(__builtin_fmaf(q, r, -x), -y, q);
+            return __builtin_fmaf(__builtin_fmaf(q, r, -x), -y, q);
+        });
+    } else {
+        body([&](float x) { return x / r; });
+    }
+}
+
 // The same row tail with one wave per row and 8 consecutive elements per lane and load
 // (rows of n % 8 == 0 values): no barrier, 16-byte loads and stores. Lane l holds chunks
 // l, l + 64, .. (J of them at most) of its row; the sums of squares run over a lane's
 // elements in order, then across the wave, so they are f32 sums in another order than
-// rows_tail_kernel's (the per-element arithmetic is the same).
+// rows_tail_kernel's (the per-element arithmetic is the same). At 2047 x 1536 values (38 MB a
+// call) 12.8 -> 9.8 us: 11.6 with the four divisions an element as refined products (two
+// waves a SIMD do not hide them), the rest from loads that no branch separates.
 template <int J>
 __global__ __launch_bounds__(256) void rows_tail_wave_kernel(TailArgs a, int n_rows) {
     const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (row >= n_rows) return;  // the whole wave
     const int C = a.n / 8;
     const size_t base = (size_t)row * a.n;
+    // Every operand of the row in flight at once, through resources of exactly the row's (the
+    // gain's) bytes: chunks past C, and operands that the mode lacks (0 bytes), read as zeros
+    // without touching memory, so no load sits behind a branch. Behind them (lanes masked by
+    // c < C, x16 and w2 by the mode) the compiler waited for each chunk's loads before it issued
+    // the next one's: six round trips a row.
+    const uint32_t fb = (uint32_t)a.n * 4, hb = (uint32_t)a.n * 2;
+    const bool norm = a.mode == G4A_TAIL_NORM || a.mode == G4A_TAIL_NORM16;
+    const rsrc_t rh = make_rsrc(a.hidden + base, fb), rx = make_rsrc(a.x16 ? a.x16 + base : nullptr, a.x16 ? hb : 0),
+                 r1 = make_rsrc(a.w1, a.x16 ? fb : 0), r2 = make_rsrc(a.w2, norm ? fb : 0);
     float8v h[J], d[J], w1[J], w2[J];
+    half8 x[J];
 #pragma unroll
-    for (int j = 0; j < J; ++j) {  // every operand of the row in flight at once
+    for (int j = 0; j < J; ++j) {
         const int c = lane + 64 * j;
-        h[j] = d[j] = w1[j] = w2[j] = float8v{};
-        if (c < C) {
-            h[j] = load8(a.hidden + base + 8 * c);
-            if (a.x16) {
-                d[j] = load8(a.x16 + base + 8 * c);
-                w1[j] = load8(a.w1 + 8 * c);
-            }
-            if (a.mode == G4A_TAIL_NORM || a.mode == G4A_TAIL_NORM16) w2[j] = load8(a.w2 + 8 * c);
-        }
-    }
-    if (a.x16) {
-        float ss = 0.0f;
-#pragma unroll
-        for (int j = 0; j < J; ++j)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                d[j][i] = srq(d[j][i], a.x_q);
-                ss = __builtin_fmaf(d[j][i], d[j][i], ss);
-            }
-        const float r = sqrtf(wave_sum(ss) / (float)a.n + a.eps);
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int c = lane + 64 * j;
-            if (c < C) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) h[j][i] = (h[j][i] + d[j][i] / r * w1[j][i]) * a.mult;
-                float* hp = a.hidden + base + 8 * c;
-                *reinterpret_cast<float4v*>(hp) = float4v{h[j][0], h[j][1], h[j][2], h[j][3]};
-                *reinterpret_cast<float4v*>(hp + 4) = float4v{h[j][4], h[j][5], h[j][6], h[j][7]};
-            }
-        }
-    }
-    if (a.mode == G4A_TAIL_NONE) return;
-    float r2 = 1.0f;
-    if (a.mode != G4A_TAIL_SRQ) {
-        float ss = 0.0f;
-#pragma unroll
-        for (int j = 0; j < J; ++j)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) ss = __builtin_fmaf(h[j][i], h[j][i], ss);
-        r2 = sqrtf(wave_sum(ss) / (float)a.n + a.eps);
+        h[j] = bload_f8(rh, 32 * c);
+        x[j] = bload_h8(rx, 16 * c);
     }
 #pragma unroll
     for (int j = 0; j < J; ++j) {
         const int c = lane + 64 * j;
-        if (c >= C) continue;
-        half8 y;
+        w1[j] = bload_f8(r1, 32 * c);
+        w2[j] = bload_f8(r2, 32 * c);
+    }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            float z = a.mode == G4A_TAIL_SRQ ? h[j][i] : pin(h[j][i] / r2 * w2[j][i]);
-            if (a.mode == G4A_TAIL_NORM16) z = (float)(half_t)z;
-            y[i] = (half_t)srq(z, a.q2);
+    for (int j = 0; j < J; ++j) d[j] = __builtin_convertvector(x[j], float8v);
+    // the arithmetic, with the quantisation steps' own forms: qx srq's the GEMM output, qy the operand
+    auto tail = [&](auto&& qx, auto&& qy) {
+        if (a.x16) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    d[j][i] = qx(d[j][i]);
+                    ss = __builtin_fmaf(d[j][i], d[j][i], ss);
+                }
+            with_quotient(sqrtf(wave_sum(ss) / (float)a.n + a.eps), [&](auto&& over) {
+#pragma unroll
+                for (int j = 0; j < J; ++j)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) h[j][i] = (h[j][i] + over(d[j][i]) * w1[j][i]) * a.mult;
+            });
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                const int c = lane + 64 * j;
+                if (c < C) {
+                    float* hp = a.hidden + base + 8 * c;
+                    *reinterpret_cast<float4v*>(hp) = float4v{h[j][0], h[j][1], h[j][2], h[j][3]};
+                    *reinterpret_cast<float4v*>(hp + 4) = float4v{h[j][4], h[j][5], h[j][6], h[j][7]};
+                }
+            }
         }
-        *reinterpret_cast<half8*>(a.y16 + base + 8 * c) = y;
+        if (a.mode == G4A_TAIL_NONE) return;
+        if (a.mode != G4A_TAIL_SRQ) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) ss = __builtin_fmaf(h[j][i], h[j][i], ss);
+            with_quotient(sqrtf(wave_sum(ss) / (float)a.n + a.eps), [&](auto&& over) {
+#pragma unroll
+                for (int j = 0; j < J; ++j)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) h[j][i] = pin(over(h[j][i]) * w2[j][i]);
+            });
+        }
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const int c = lane + 64 * j;
+            if (c >= C) continue;
+            half8 y;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                float z = h[j][i];
+                if (a.mode == G4A_TAIL_NORM16) z = (float)(half_t)z;
+                y[i] = (half_t)qy(z);
+            }
+            *reinterpret_cast<half8*>(a.y16 + base + 8 * c) = y;
+        }
+    };
+    if ((!a.x16 || srq_fast(a.x_q)) && (a.mode == G4A_TAIL_NONE || srq_fast(a.q2))) {
+        const SrqStep tx = srq_step(a.x16 ? a.x_q : 1.0f), ty = srq_step(a.mode == G4A_TAIL_NONE ? 1.0f : a.q2);
+        tail([&](float x) { return pin(srq_index(x, tx) * tx.s); }, [&](float x) { return pin(srq_index(x, ty) * ty.s); });
+    } else {
+        tail([&](float x) { return srq(x, a.x_q); }, [&](float x) { return srq(x, a.q2); });
     }
 }
 
