@@ -37,7 +37,7 @@ struct PrefillArgs {
     void* out;
     int S, start_pos, n_q_heads, n_kv_heads, window, n_qblocks;
     float scale_log2, eps, out_q;
-    // key split of long causal rows (prefill_kernel_w32): split_tiles = 0 means none;
+    // key split of long causal rows: split_tiles = 0 means none;
     // otherwise a workgroup covers at most split_tiles key tiles of its query block and
     // blocks with more tiles leave partials for prefill_merge_kernel
     int split_tiles, max_pieces, pieces_per_head;
@@ -278,8 +278,11 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32(PrefillArgs a) {
     const int n_tiles = (kv_hi - wg_lo + KT - 1) / KT;
     int t0 = 0, t1 = n_tiles;
     if (a.split_tiles > 0) {
-        t0 = piece * a.split_tiles;
-        t1 = min(t0 + a.split_tiles, n_tiles);
+        // even shares, none above split_tiles, the longer ones first: the last holds the diagonal
+        // (S 1024, 16 tiles in 6 pieces: 24.6 us a call; longer ones spread out 25.5)
+        const int share = n_tiles / n_pieces, longer = n_tiles - share * n_pieces;
+        t0 = piece * share + min(piece, longer);
+        t1 = t0 + share + (piece < longer);
     }
 
     // ---- this lane's query column (head hh, position offset pl) and 8-dim half h
@@ -745,8 +748,10 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32d(PrefillArgs a) {
     const int n_tiles = (kv_hi - wg_lo + KT - 1) / KT;
     int t0 = 0, t1 = n_tiles;
     if (a.split_tiles > 0) {
-        t0 = piece * a.split_tiles;
-        t1 = min(t0 + a.split_tiles, n_tiles);
+        // even shares, none above split_tiles; the last one, on the diagonal, is the
+        // shorter; longer ones spread out (S 1900 after 1100 150 us, longer ones first 155)
+        t0 = (piece * n_tiles + n_pieces - 1) / n_pieces;
+        t1 = ((piece + 1) * n_tiles + n_pieces - 1) / n_pieces;
     }
 
     // ---- this lane's query column (head hh, position offset pl) and 8-dim half h
@@ -1049,8 +1054,10 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32h(PrefillArgs a) {
     const int n_tiles = (kv_hi - wg_lo + KT - 1) / KT;
     int t0 = 0, t1 = n_tiles;
     if (a.split_tiles > 0) {
-        t0 = piece * a.split_tiles;
-        t1 = min(t0 + a.split_tiles, n_tiles);
+        // even shares, none above split_tiles; the last one, on the diagonal, is the
+        // shorter; longer ones spread out (S 1900 after 1100 150 us, longer ones first 155)
+        t0 = (piece * n_tiles + n_pieces - 1) / n_pieces;
+        t1 = ((piece + 1) * n_tiles + n_pieces - 1) / n_pieces;
     }
 
     // ---- this lane's query column (head hh, position offset pl) and 8-dim half h
@@ -1455,10 +1462,14 @@ static prefill_fn pick_g(int G, bool out32, bool hilo, bool klo, bool split) {
 using namespace g4a;
 
 // Key split for short prompts: when the query blocks alone give fewer than 2 workgroups
-// per CU, long causal rows are cut into pieces of split_tiles key tiles, the longest block
-// into about six pieces. Measured best piece sizes at 16 / 24 / 32 / 64 tiles in the
-// longest block (S 1024, 1536, 2048, 4096 global): 3 / 3-4 / 5 / 10-13 tiles; one piece
-// per CU (3 / 5 / 9 / 33) was up to 24 % slower beyond S 1024.
+// per CU, long causal rows are cut into even pieces of at most split_tiles key tiles, the
+// longest block into 2 to 7 of them: as many as fill whole rounds of one piece a CU. Against
+// always about six pieces with the remainder in the last: hd 512 (f16 q, 1 KV head) S 1900
+// after 1100 187 -> 150 us a call, S 2047 108 -> 101, S 4096 321 -> 287; hd 256 (2 KV heads)
+// S 1500 40.3 -> 33.7, S 3000 82 -> 74; q and caches in f32, hd 256 S 1500 62 -> 53, hd 512
+// S 700 54 -> 43, S 2047 165 -> 148; relative rms error against f64 1.97e-4 -> 1.90e-4 (hd 256
+// S 1500), 2.91e-4 before and after (hd 512 S 1900). Where that rule already gave one round (hd 256 S 1024,
+// S 600 after 3000; hd 512 S 1024) the plan is the same.
 struct PrefillSplit {
     int split_tiles, max_pieces, n_qblocks, total_pieces;
     int kv_row0, kv_rows;  // f32 caches: the attended rows copied to f16
@@ -1508,6 +1519,7 @@ static PrefillSplit prefill_split(const g4a_cfg* cfg, int S, int start_pos) {
         const int nt = (hi - lo + KT - 1) / KT;
         if (nt > max_tiles) max_tiles = nt;
     }
+    // the workspace: about six pieces of the longest block
     int st = (max_tiles * 5 + 31) / 32;
     // at least 2 tiles a piece, 4 for prefill_kernel_w32h's 32-key tiles (hd 512, S 1024,
     // W 512, 17-tile blocks: 3 tiles a piece 53.5 us a call, 4 tiles 43.4, 5 tiles 47.4;
@@ -1515,8 +1527,30 @@ static PrefillSplit prefill_split(const g4a_cfg* cfg, int S, int start_pos) {
     const int st_min = HD == 512 && NCOL == 128 ? 4 : 2;
     if (st < st_min) st = st_min;
     if (st < (max_tiles + 7) / 8) st = (max_tiles + 7) / 8;  // the merge takes <= 8 pieces
-    const int pieces = (max_tiles + st - 1) / st;
-    if (pieces <= 1) return p;
+    const int room = (max_tiles + st - 1) / st;  // the workspace holds this many pieces a block
+    if (room <= 1) return p;
+    // of the piece counts that the workspace holds, the one whose rounds of 256 workgroups (one
+    // a CU) end first: a round lasts its longest piece, step us a tile and fixed us a piece.
+    // Measured, us a call (rounds x tiles): hd 512, S 1900 after 1100, 94-tile blocks: 3 x 16
+    // 180, 3 x 14 166, 2 x 24 175, 2 x 19 151, 1 x 47 164; S 2047, 64 tiles: 2 x 10 100, 2 x 16
+    // 128, 1 x 22 98; hd 256, S 3000, 2 KV heads, 47 tiles: 3 x 8 81, 2 x 12 74, 2 x 16 84
+    const float step = HD == 256 ? 1.5f : 3.0f, fixed = HD == 256 ? 7.0f : 5.0f;
+    int pieces = room;
+    float best = 0.0f;
+    for (int n = 2; n <= room; ++n) {
+        int tiles = (max_tiles + n - 1) / n, wgs = 0;
+        if (tiles < st_min) tiles = st_min;
+        for (int t = 0; t < max_tiles; t += tiles) {  // blocks of more than t tiles
+            const int beyond = t * KT - start_pos;
+            if (W == 0 || t == 0 || t * KT < BQ + W - 1) wgs += p.n_qblocks - (beyond > 0 ? beyond / BQ : 0);
+        }
+        const float us = (float)((wgs * kvH + 255) / 256) * (tiles * step + fixed);
+        if (n == 2 || us < best) {
+            best = us;
+            st = tiles;
+            pieces = (max_tiles + tiles - 1) / tiles;
+        }
+    }
     p.split_tiles = st;
     p.max_pieces = pieces;
     p.total_pieces = 0;
@@ -1527,7 +1561,7 @@ static PrefillSplit prefill_split(const g4a_cfg* cfg, int S, int start_pos) {
         const int nt = (hi - lo + KT - 1) / KT;
         p.total_pieces += nt > st ? (nt + st - 1) / st : 1;
     }
-    const size_t slots = (size_t)kvH * p.n_qblocks * pieces * NCOL;
+    const size_t slots = (size_t)kvH * p.n_qblocks * room * NCOL;
     p.q16_bytes = q16;
     p.q16lo_bytes = hilo ? q16 : 0;
     p.o_bytes = slots * HD * sizeof(half_t);
