@@ -419,8 +419,12 @@ struct TileCfg {
 constexpr TileCfg kTiles[] = {{256, 256, 1.45f, 7.0f, 0}, {256, 192, 1.15f, 6.0f, 1}, {192, 128, 0.68f, 5.0f, 1},
                               {128, 128, 0.45f, 4.5f, 1}, {64, 128, 0.30f, 4.0f, 1}};
 constexpr int kFirstSplit = 3;  // the tiles that have a split form
-// A split adds the tile's partials through memory: about 3 us, and 0.8 us for each of them.
-constexpr float kMergeFixed = 3.0f, kMergeEach = 0.8f;
+// A split adds the tile's partials through memory: 0.25 us for each of a tile's and 0.03 us for
+// each workgroup of the launch, a fit to 64x128 and 128x128 splits of 2 to 8 at M 1 to 2047,
+// K 1536 to 12288 (the plan is within 5 % of the fastest tile and split of all 66 products; a
+// flat 3 + 0.8 us a split was up to 25 % off): N 256 K 1536 M 1 9.2 -> 7.6 us, M 1024 10.3 ->
+// 9.6; N 1536 K 2048 M 300 14.0 -> 11.5.
+constexpr float kMergeEach = 0.25f, kMergeGroup = 0.03f;
 
 // The workspace contract (g4a_gemm16_ws_bytes): launches of fewer 128 x 64 output tiles than
 // CUs may split k up to `max_splits` times, at least four k-stages each, and are asked for that
@@ -456,7 +460,7 @@ GemmPlan gemm_plan(int M, int K, int n_mats, const int* rows, int max_splits) {
         for (int i = 0; i < n_mats; ++i) tiles += (long)((rows[i] + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm);
         for (int s = 1; s <= (c >= kFirstSplit && tiles <= (long)(kTicketBytes / 4) ? max_splits : 1); ++s) {
             const long rounds = (tiles * s + kCUs - 1) / kCUs;
-            const float cost = rounds * ((K / 64 + s - 1) / s * t.step + t.fixed) + (s > 1 ? kMergeFixed + kMergeEach * s : 0.0f);
+            const float cost = rounds * ((K / 64 + s - 1) / s * t.step + t.fixed) + (s > 1 ? kMergeEach * s + kMergeGroup * (tiles * s) : 0.0f);
             if (!best.tiles || cost < least) {
                 best = {c, (int)tiles, s};
                 least = cost;

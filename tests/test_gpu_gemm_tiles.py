@@ -57,7 +57,8 @@ def test_every_tile_matches_float64(M, K, ns):
     assert torch.equal(q[:M], want) and (q[M:] == 7.0).all()
 
 
-@pytest.mark.parametrize("M,K,ns", [(77, 4096, (128, 384)), (1, 8192, (128,)), (1000, 12288, (1536,)), (130, 6144, (1536,))])
+@pytest.mark.parametrize("M,K,ns", [(77, 4096, (128, 384)), (1, 8192, (128,)), (1000, 12288, (1536,)), (130, 6144, (1536,)),
+                                    (40, 1024, (128,)), (200, 1344, (256,)), (300, 2048, (1536,)), (1, 1536, (256,))])
 def test_split_tiles_match_float64_and_repeat(M, K, ns):
     print(f"gemm16 split M {M} K {K} n {ns}", flush=True)
     a, ws = operands(M, K, ns, M + K)
