@@ -27,6 +27,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "gemm_offsets.hpp"
 
 namespace g4a {
 
@@ -111,7 +112,7 @@ enum GemmMode { kPlain, kSplitK, kGeglu };
 template <int BM, int BN, int WM, int WN, int ST, int MINW, GemmMode MODE>
 __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm16_kernel(Gemm16Args g) {
     constexpr int NW = WM * WN, TM = BM / WM, TN = BN / WN, MB = TM / 32, NB = TN / 32;
-    constexpr int ROWB = 128, STB = (BM + BN) * ROWB;
+    constexpr int ROWB = kStageBytes, STB = (BM + BN) * ROWB;
     constexpr int DW = BN / 8 / NW, DA = BM / 8 / NW, D = DW + DA;  // 1 KiB DMAs per wave and stage
     static_assert(TM % 32 == 0 && TN % 32 == 0 && DW * 8 * NW == BN && DA * 8 * NW == BM, "even shares");
     static_assert(ST >= 2 && (ST - 1) * D < 64 && ST * STB <= 160 * 1024, "vmcnt holds 6 bits; LDS holds 160 KiB");
@@ -162,21 +163,18 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm16_kernel(Gemm16Args g
         const int r = 8 * (wave * DA + j) + lane / 8;
         va[j] = (m0 + r) * K * 2 + 16 * ((lane % 8) ^ swz(r));
     }
-    // DMA d of k-stage t into buffer buf; more = 0: past the range, an empty resource (no memory
-    // is read and zeros go into a buffer that nobody reads any more)
+    // DMA d of k-stage t into buffer buf; more = 0: past the range, an empty resource at offset 0 (no
+    // memory is read and zeros go into a buffer that nobody reads any more)
     auto dma = [&](auto dc, int t, int buf, bool more) {
         constexpr int d = decltype(dc)::value;
-        const int soff = (kt0 + t) * ROWB;
         const uint32_t b = lbase + buf * STB;
-        if constexpr (d < DW) {
-            int4v q = GEGLU && ((wave * DW + d) / 2) % 2 ? ru : rw;
-            q[2] = more ? q[2] : 0;
-            dma16(q, vw[d], soff, b + (wave * DW + d) * 1024);
-        } else {
-            int4v q = ra;
-            q[2] = more ? q[2] : 0;
-            dma16(q, va[d - DW], soff, b + BN * ROWB + (wave * DA + d - DW) * 1024);
-        }
+        int4v q = d >= DW ? ra : GEGLU && ((wave * DW + d) / 2) % 2 ? ru : rw;
+        const StageDma at = stage_dma((uint32_t)q[2], kt0 + t, more);
+        q[2] = (int)at.records;
+        if constexpr (d < DW)
+            dma16(q, vw[d], (int)at.soff, b + (wave * DW + d) * 1024);
+        else
+            dma16(q, va[d - DW], (int)at.soff, b + BN * ROWB + (wave * DA + d - DW) * 1024);
     };
 
     float lut_entry = 0.0f;  // out before the stages, used after them
