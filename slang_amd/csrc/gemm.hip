@@ -78,7 +78,7 @@ __device__ __forceinline__ int4v rsrc4(const void* p, uint32_t bytes) {
 }
 // 16 bytes a lane from rs + voff + soff to LDS address lds + 16 lane. No output register: the
 // data is in LDS once vmcnt has counted it (wait_barrier).
-__device__ __forceinline__ void dma16(int4v rs, int voff, int soff, uint32_t lds) {
+__device__ __forceinline__ void dma16(int4v rs, uint32_t voff, uint32_t soff, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs),
                  "s"(soff));
 }
@@ -151,17 +151,17 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm16_kernel(Gemm16Args g
     // rows an instruction; rows past M or N read as zeros
     const int4v ra = rsrc4(g.a, (uint32_t)g.M * K * 2), rw = rsrc4(g.w[p], (uint32_t)N * K * 2);
     const int4v ru = GEGLU ? rsrc4(g.w[1], (uint32_t)N * K * 2) : rw;
-    int vw[DW], va[DA];
+    uint32_t vw[DW], va[DA];
 #pragma unroll
     for (int j = 0; j < DW; ++j) {
         const int i = wave * DW + j, r = 8 * i + lane / 8;
         const int row = n0 + (GEGLU ? 16 * (i / 4) + r % 16 : r);
-        vw[j] = row * K * 2 + 16 * ((lane % 8) ^ swz(r));
+        vw[j] = row_offset(row, K) + 16 * ((lane % 8) ^ swz(r));
     }
 #pragma unroll
     for (int j = 0; j < DA; ++j) {
         const int r = 8 * (wave * DA + j) + lane / 8;
-        va[j] = (m0 + r) * K * 2 + 16 * ((lane % 8) ^ swz(r));
+        va[j] = row_offset(m0 + r, K) + 16 * ((lane % 8) ^ swz(r));
     }
     // DMA d of k-stage t into buffer buf; more = 0: past the range, an empty resource at offset 0 (no
     // memory is read and zeros go into a buffer that nobody reads any more)
@@ -172,9 +172,9 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm16_kernel(Gemm16Args g
         const StageDma at = stage_dma((uint32_t)q[2], kt0 + t, more);
         q[2] = (int)at.records;
         if constexpr (d < DW)
-            dma16(q, vw[d], (int)at.soff, b + (wave * DW + d) * 1024);
+            dma16(q, vw[d], at.soff, b + (wave * DW + d) * 1024);
         else
-            dma16(q, va[d - DW], (int)at.soff, b + BN * ROWB + (wave * DA + d - DW) * 1024);
+            dma16(q, va[d - DW], at.soff, b + BN * ROWB + (wave * DA + d - DW) * 1024);
     };
 
     float lut_entry = 0.0f;  // out before the stages, used after them

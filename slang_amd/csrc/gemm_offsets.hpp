@@ -18,4 +18,9 @@ constexpr StageDma stage_dma(uint32_t bytes, int stage, bool more) {
     return more ? StageDma{bytes, (uint32_t)stage * kStageBytes} : StageDma{0, 0};
 }
 
+// Byte offset of row `row` of a matrix of rows of K f16 values. A tile's rows past the matrix reach
+// up to 255 rows beyond it, past 2^31 where the matrix ends just below (the launch checks leave 127
+// rows), but never past 2^32: they read as zeros.
+constexpr uint32_t row_offset(int row, int K) { return (uint32_t)row * (uint32_t)K * 2u; }
+
 }  // namespace g4a

@@ -47,3 +47,34 @@ constexpr bool check() {
 }
 static_assert(check(), "a DMA out of its matrix's k-stages");
 """)
+
+
+def test_row_offsets_at_the_ends_of_what_is_accepted(tmp_path):
+    """Rows of a tile past the matrix get offsets past its bytes: formed in 32 bits they neither
+    overflow nor wrap back into it, for every tile height (tokens to 256; weight rows to 256, the
+    gate/up form's outputs to 128) and the largest K and row counts that g4a_gemm16 and
+    g4a_gemm16_geglu take: (M + 127) K 2 and n K 2 up to 2^31 - 1, n in steps of 128 (64)."""
+    holds(tmp_path, """
+constexpr uint64_t kMost = 0x7fffffff;
+constexpr bool rows_ok(uint64_t rows, uint64_t K, uint64_t tile) {
+    const uint64_t bytes = rows * K * 2, end = (rows + tile - 1) / tile * tile;
+    for (uint64_t r = rows > 2 ? rows - 2 : 0; r < end; ++r) {
+        const uint64_t off = row_offset((int)r, (int)K) + (uint64_t)(kStageBytes - 16), exact = r * K * 2 + kStageBytes - 16;
+        if (off != exact || (r >= rows && off < bytes) || off + K * 2 > 0xffffffffu) return false;
+    }
+    return true;
+}
+constexpr bool check() {
+    for (uint64_t tile : {64, 96, 128, 192, 256})
+        for (uint64_t K = 64; K * 2 * 128 <= kMost; K *= 2) {
+            for (uint64_t k : {K, K * 2 - 64}) {
+                if (k * 2 * 128 > kMost) continue;
+                if (!rows_ok(kMost / (k * 2) - 127, k, tile) || !rows_ok(1, k, tile)) return false;
+                if (!rows_ok(kMost / (k * 2) / 128 * 128, k, tile)) return false;
+                if (tile <= 128 && !rows_ok(kMost / (k * 2) / 64 * 64, k, tile)) return false;
+            }
+        }
+    return true;
+}
+static_assert(check(), "an offset that wraps");
+""")
