@@ -23,9 +23,14 @@
 // the f16 pair (q_hi, q_lo) (G4A_Q_HILO, attn_prefill's f32 q). f32 caches (G4A_KV_F32) are
 // converted to f16 as the GEMM form's srqh_b does, and with G4A_Q_HILO (attn_prefill on its
 // own f32 caches) K is kept as the f16 pair (k_hi, k_lo), so the scores are f32-accurate.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace g4a {
+
+typedef unsigned v4u32 __attribute__((ext_vector_type(4)));
+typedef unsigned v2u32 __attribute__((ext_vector_type(2)));
 
 struct PrefillArgs {
     const float* q;
@@ -39,34 +44,95 @@ struct PrefillArgs {
     float scale_log2, eps, out_q;
     // key split of long causal rows: split_tiles = 0 means none;
     // otherwise a workgroup covers at most split_tiles key tiles of its query block and
-    // blocks with more tiles leave partials for prefill_merge_kernel
-    int split_tiles, max_pieces, pieces_per_head;
+    // blocks with more tiles leave partials for prefill_merge_kernel (part24: in 24 bits a value)
+    int split_tiles, max_pieces, pieces_per_head, part24;
     int xcd_runs;  // prefill_kernel_w32 unsplit: 1-D grid, query blocks in contiguous runs per XCD
     int xcd_heads;  // unsplit causal: 1-D grid, kv head h on XCDs 8h/kvH .., its blocks longest first
     const half_t* q16;  // prefill_kernel_w32: q already prepared in f16 (qprep_kernel), or NULL
     const half_t* q16lo;  // ... and with G4A_Q_HILO its f16 low parts (q - f32(q16))
     int kv_row0;  // prefill_kernel_w32: first row held in kc/vc (rows below it are never read)
     const void* kclo;  // f32 caches: the f16 low parts k - f32(f16(k)) of the f16 K copy in kc
-    half_t* part_o;   // [kvH][n_qblocks][max_pieces] blocks of NCOL x HD O / l in f16, in the
-                      // accumulator layout [wave block][dt][j pair][lane][8] (see prefill_merge_kernel)
-    float2* part_ml;  // [kvH][n_qblocks][max_pieces][128 columns] (m, l)
+    // The pieces' O / l, blocks of NCOL x HD values, and their (m, l), NCOL pairs a block. f16 values
+    // in the accumulator layout [wave block][dt][j pair][lane][8] (prefill_merge_kernel), a block a
+    // [kvH][n_qblocks][max_pieces]. part24: the upper halves of its f32 values in that layout,
+    // then their third bytes in the same order, a block a [kvH][pieces_per_head] in the work
+    // list's order: with short blocks' absent pieces left out, more of these larger blocks fit.
+    void* part_o;
+    float2* part_ml;
 };
+
+constexpr int kMaxPieces24 = 5;  // pieces of a block with part24
 
 // Most a column's running maximum lags its true maximum by (log2 units): P <= 2^15 < 65504
 constexpr float kMaxLag = 15.0f;
 
-// Rows j0 .. j0 + 7 of a 32x32 accumulator tile (two 4-row groups of one lane) times inv,
-// as one 16-byte f16 store: the split pieces' partial O. NT: on the non-temporal policy,
-// which the hd-256 pieces take (their 12 MB of partials at S 1024, with the q rows also
-// stored that way: config 3G 27.2 -> 26.5 us, 3S 25.2 -> 25.55 us) and the hd-512 ones do
-// not (29 MB: 47.3 -> 49.2 us).
-template <bool NT, typename ACC>
-__device__ __forceinline__ void store_part8(half_t* dst, const ACC& acc, int j0, float inv) {
-    half8 v;
+// The tile range [t0, t1) of piece `piece` of a block of n_tiles. f16 partials: split_tiles each,
+// the rest in the last. part24: even shares, none above split_tiles.
+struct PieceTiles {
+    int t0, t1;
+};
+__device__ __forceinline__ PieceTiles piece_tiles(const PrefillArgs& a, bool part24, int piece, int n_pieces, int n_tiles) {
+    if (a.split_tiles == 0) return PieceTiles{0, n_tiles};
+    if (part24) return PieceTiles{(piece * n_tiles + n_pieces - 1) / n_pieces, ((piece + 1) * n_tiles + n_pieces - 1) / n_pieces};
+    return PieceTiles{piece * a.split_tiles, min((piece + 1) * a.split_tiles, n_tiles)};
+}
+
+// f32 values rounded to their upper 24 bits (a 16-bit mantissa, 2^-17 relative; an infinity and
+// the NaNs that f16 operands make keep their bits), eight at a time: the upper halves, and the
+// third bytes.
+struct Part24 {
+    v4u32 hi;
+    v2u32 lo;
+};
+template <typename ACC>
+__device__ __forceinline__ Part24 pack24(const ACC& acc, int j0, float inv) {
+    uint32_t x[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = (half_t)(acc[j0 + i] * inv);
-    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<half8*>(dst));
-    else *reinterpret_cast<half8*>(dst) = v;
+    for (int i = 0; i < 8; ++i) x[i] = __builtin_bit_cast(uint32_t, acc[j0 + i] * inv) + 0x80u;
+    Part24 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.hi[i] = __builtin_amdgcn_perm(x[2 * i + 1], x[2 * i], 0x07060302);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t p0 = __builtin_amdgcn_perm(x[4 * i + 1], x[4 * i], 0x0c0c0501);
+        const uint32_t p1 = __builtin_amdgcn_perm(x[4 * i + 3], x[4 * i + 2], 0x0c0c0501);
+        r.lo[i] = __builtin_amdgcn_perm(p1, p0, 0x05040100);
+    }
+    return r;
+}
+// value i of the eight
+__device__ __forceinline__ float unpack24(v4u32 hi, v2u32 lo, int i) {
+    const uint32_t sel = (i & 1 ? 0x07060000u : 0x05040000u) | (uint32_t)(i & 3) << 8 | 0x0cu;
+    return __builtin_bit_cast(float, __builtin_amdgcn_perm(hi[i / 2], lo[i / 4], sel));
+}
+
+// The partial of one 32x32 accumulator tile dt of wave block w (of 32 x DIMS), times inv, as
+// contiguous runs of all 64 lanes, into the piece's block `slot` of NV = NCOL x HD values. NT: on the
+// non-temporal policy, which the hd-256 pieces take (their 12 MB of partials at S 1024, with the q
+// rows also stored that way: config 3G 27.2 -> 26.5 us, 3S 25.2 -> 25.55 us) and the hd-512 ones
+// do not (29 MB: 47.3 -> 49.2 us).
+template <bool NT, int DIMS, int NV, typename ACC>
+__device__ __forceinline__ void store_part(void* part_o, bool part24, int slot, int w, int dt, int lane, const ACC& acc, float inv) {
+    char* base = reinterpret_cast<char*>(part_o) + (size_t)slot * (NV * (part24 ? 3 : 2));
+    const int run0 = w * (32 * DIMS) + dt * 1024;
+    auto put = [](auto* dst, auto v) {
+        if constexpr (NT) __builtin_nontemporal_store(v, dst);
+        else *dst = v;
+    };
+#pragma unroll
+    for (int jp = 0; jp < 2; ++jp) {
+        const int run = run0 + 512 * jp + 8 * lane;
+        if (part24) {
+            const Part24 v = pack24(acc, 8 * jp, inv);
+            put(reinterpret_cast<v4u32*>(base + 2 * run), v.hi);
+            put(reinterpret_cast<v2u32*>(base + 2 * NV + run), v.lo);
+        } else {
+            half8 v;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = (half_t)(acc[8 * jp + i] * inv);
+            put(reinterpret_cast<half8*>(base + 2 * run), v);
+        }
+    }
 }
 
 // LDS operand reads issued ahead of their MFMAs in prefill_kernel_w32: score product
@@ -199,18 +265,17 @@ __device__ __forceinline__ int vswz(int r) { return (0x6CA0 >> (4 * (r & 3))) & 
 // blocks at a time (one division each, in parallel) and a prefix sum over the wave finds the
 // block holding piece i; a scalar loop over the blocks would cost microseconds of issue slots.
 struct PrefillUnit {
-    int kh, qb, piece, n_pieces;
+    int kh, qb, piece, n_pieces, slot;
 };
+// pieces of query block b: its keys [lo(b), hi(b)) in tiles of KT keys, split_tiles a piece
+__device__ __forceinline__ int block_pieces(const PrefillArgs& a, int b, int BQ, int KT) {
+    const int b0 = a.start_pos + b * BQ;
+    const int hi = min(b0 + BQ, a.start_pos + a.S), lo = a.window > 0 ? max(0, b0 + 1 - a.window) : 0;
+    return max(1, ((hi - lo + KT - 1) / KT + a.split_tiles - 1) / a.split_tiles);
+}
 template <int BQ, int KT>
 __device__ __forceinline__ PrefillUnit prefill_unit(const PrefillArgs& a, int lane) {
-    const int T_total = a.start_pos + a.S;
-    // key tiles of query block b: [lo(b), hi(b)) in tiles of KT keys
-    auto block_tiles = [&](int b) {
-        const int b0 = a.start_pos + b * BQ;
-        const int hi = min(b0 + BQ, T_total), lo = a.window > 0 ? max(0, b0 + 1 - a.window) : 0;
-        return (hi - lo + KT - 1) / KT;
-    };
-    int kh = blockIdx.y, qb = a.n_qblocks - 1 - (int)blockIdx.x, piece = 0, n_pieces = 1;
+    int kh = blockIdx.y, qb = a.n_qblocks - 1 - (int)blockIdx.x, piece = 0, n_pieces = 1, slot = 0;
     if (a.xcd_heads) {
         // causal, unsplit: kv head kh on its own 8/kvH XCDs (the dispatcher deals workgroup L
         // to XCD L % 8), each head's blocks longest first across them
@@ -233,7 +298,7 @@ __device__ __forceinline__ PrefillUnit prefill_unit(const PrefillArgs& a, int la
         int base = 0;  // pieces of the blocks before this group of 64
         for (int k0 = 0; k0 < a.n_qblocks; k0 += 64) {
             const int b = a.n_qblocks - 1 - (k0 + lane);
-            const int np = b >= 0 ? max(1, (block_tiles(b) + a.split_tiles - 1) / a.split_tiles) : 0;
+            const int np = b >= 0 ? block_pieces(a, b, BQ, KT) : 0;
             const int incl = wave_prefix_sum(np);
             const unsigned long long past = __ballot(base + incl > i);  // lanes whose range ends past piece i
             if (past) {
@@ -245,11 +310,12 @@ __device__ __forceinline__ PrefillUnit prefill_unit(const PrefillArgs& a, int la
             }
             base += __builtin_amdgcn_readlane(incl, 63);
         }
+        slot = a.part24 ? v : (kh * a.n_qblocks + qb) * a.max_pieces + piece;
     }
-    return PrefillUnit{kh, qb, piece, n_pieces};
+    return PrefillUnit{kh, qb, piece, n_pieces, slot};
 }
 
-template <int G, typename OUTT, bool HILO, bool KLO, bool SPLITK>
+template <int G, typename OUTT, bool HILO, bool KLO, bool SPLITK, bool P24>
 __global__ __launch_bounds__(256) void prefill_kernel_w32(PrefillArgs a) {
     constexpr int HD = 256, KT = 64, NCOL = 128, BQ = NCOL / G;
     constexpr int QMF = HILO ? 2 : 1;  // score MFMAs per K operand (q high, then low parts)
@@ -276,14 +342,8 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32(PrefillArgs a) {
     const int kv_hi = min(p0 + BQ, T_total);
     const int wg_lo = a.window > 0 ? max(0, p0 + 1 - a.window) : 0;
     const int n_tiles = (kv_hi - wg_lo + KT - 1) / KT;
-    int t0 = 0, t1 = n_tiles;
-    if (a.split_tiles > 0) {
-        // even shares, none above split_tiles, the longer ones first: the last holds the diagonal
-        // (S 1024, 16 tiles in 6 pieces: 24.6 us a call; longer ones spread out 25.5)
-        const int share = n_tiles / n_pieces, longer = n_tiles - share * n_pieces;
-        t0 = piece * share + min(piece, longer);
-        t1 = t0 + share + (piece < longer);
-    }
+    const PieceTiles tiles = piece_tiles(a, P24, piece, n_pieces, n_tiles);
+    const int t0 = tiles.t0, t1 = tiles.t1;
 
     // ---- this lane's query column (head hh, position offset pl) and 8-dim half h
     const int c = 32 * wave + n32;
@@ -660,16 +720,11 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32(PrefillArgs a) {
 
     // ---- epilogue: column sum over both halves, normalise, srq, store 4 dims at a time
     const float l_tot = add32(l_run);
-    if (SPLITK && n_pieces > 1) {  // a piece of a split query block: O / l in f16 and (m, l) in f32
-        const size_t blk = ((size_t)kh * a.n_qblocks + qb) * a.max_pieces + piece;
+    if (SPLITK && n_pieces > 1) {  // a piece of a split query block: O / l and (m, l)
         const float inv_p = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-        // one 1 KiB run per store instruction: [wave][dt][j pair][lane] half8
-        half_t* po = a.part_o + blk * (NCOL * HD) + (size_t)wave * (32 * HD) + 8 * lane;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-            for (int jp = 0; jp < 2; ++jp) store_part8<true>(po + (2 * dt + jp) * 512, oacc[dt], 8 * jp, inv_p);
-        if (h == 0) a.part_ml[blk * NCOL + c] = make_float2(m_use, l_tot);
+        for (int dt = 0; dt < 8; ++dt) store_part<true, HD, NCOL * HD>(a.part_o, P24, wu.slot, wave, dt, lane, oacc[dt], inv_p);
+        if (h == 0) a.part_ml[(size_t)wu.slot * NCOL + c] = make_float2(m_use, l_tot);
         return;
     }
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
@@ -746,13 +801,8 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32d(PrefillArgs a) {
     const int kv_hi = min(p0 + BQ, T_total);
     const int wg_lo = a.window > 0 ? max(0, p0 + 1 - a.window) : 0;
     const int n_tiles = (kv_hi - wg_lo + KT - 1) / KT;
-    int t0 = 0, t1 = n_tiles;
-    if (a.split_tiles > 0) {
-        // even shares, none above split_tiles; the last one, on the diagonal, is the
-        // shorter; longer ones spread out (S 1900 after 1100 150 us, longer ones first 155)
-        t0 = (piece * n_tiles + n_pieces - 1) / n_pieces;
-        t1 = ((piece + 1) * n_tiles + n_pieces - 1) / n_pieces;
-    }
+    const PieceTiles tiles = piece_tiles(a, a.part24, piece, n_pieces, n_tiles);
+    const int t0 = tiles.t0, t1 = tiles.t1;
 
     // ---- this lane's query column (head hh, position offset pl) and 8-dim half h
     const int c = 32 * pr + n32;
@@ -969,15 +1019,11 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32d(PrefillArgs a) {
 
     // ---- epilogue: this wave's 256 dims of its 32 columns
     const float l_tot = add32(l_run);
-    if (n_pieces > 1) {  // a piece of a split query block: O / l in f16, (m, l) from wave dh 0
-        const size_t blk = ((size_t)kh * a.n_qblocks + qb) * a.max_pieces + piece;
+    if (n_pieces > 1) {  // a piece of a split query block: O / l, (m, l) from wave dh 0
         const float inv_p = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-        half_t* po = a.part_o + blk * (NCOL * HD) + (size_t)wave * (32 * 256) + 8 * lane;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-            for (int jp = 0; jp < 2; ++jp) store_part8<false>(po + (2 * dt + jp) * 512, oacc[dt], 8 * jp, inv_p);
-        if (h == 0 && dh == 0) a.part_ml[blk * NCOL + c] = make_float2(m_use, l_tot);
+        for (int dt = 0; dt < 8; ++dt) store_part<false, 256, NCOL * HD>(a.part_o, a.part24, wu.slot, wave, dt, lane, oacc[dt], inv_p);
+        if (h == 0 && dh == 0) a.part_ml[(size_t)wu.slot * NCOL + c] = make_float2(m_use, l_tot);
         return;
     }
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
@@ -1032,7 +1078,7 @@ __device__ __forceinline__ void mfma32_acc(float16v& acc, half8 a, half8 b) {
     asm("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
-template <int G, typename OUTT, bool QSTAGE, bool OSTAGE>
+template <int G, typename OUTT, bool QSTAGE, bool OSTAGE, bool P24>
 __global__ __launch_bounds__(256) void prefill_kernel_w32h(PrefillArgs a) {
     constexpr int HD = 512, KT = 32, NCOL = 128, BQ = NCOL / G;
     constexpr int ROWB = HD * 2;      // 1 KiB rows
@@ -1052,13 +1098,8 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32h(PrefillArgs a) {
     const int kv_hi = min(p0 + BQ, T_total);
     const int wg_lo = a.window > 0 ? max(0, p0 + 1 - a.window) : 0;
     const int n_tiles = (kv_hi - wg_lo + KT - 1) / KT;
-    int t0 = 0, t1 = n_tiles;
-    if (a.split_tiles > 0) {
-        // even shares, none above split_tiles; the last one, on the diagonal, is the
-        // shorter; longer ones spread out (S 1900 after 1100 150 us, longer ones first 155)
-        t0 = (piece * n_tiles + n_pieces - 1) / n_pieces;
-        t1 = ((piece + 1) * n_tiles + n_pieces - 1) / n_pieces;
-    }
+    const PieceTiles tiles = piece_tiles(a, P24, piece, n_pieces, n_tiles);
+    const int t0 = tiles.t0, t1 = tiles.t1;
 
     // ---- this lane's query column (head hh, position offset pl) and 8-dim half h
     const int c = 32 * wave + n32;
@@ -1291,17 +1332,13 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32h(PrefillArgs a) {
                    "+a"(oacc[6]), "+a"(oacc[7]), "+a"(oacc[8]), "+a"(oacc[9]), "+a"(oacc[10]), "+a"(oacc[11]),
                    "+a"(oacc[12]), "+a"(oacc[13]), "+a"(oacc[14]), "+a"(oacc[15]));
     const float l_tot = add32(l_run);
-    if (n_pieces > 1) {  // a piece of a split query block: O / l in f16 and (m, l) in f32
-        // blocks of 32 columns x 256 dims, [wave][dim half][dt % 8][j pair][lane] half8: the
+    if (QSTAGE && n_pieces > 1) {  // a piece of a split query block: O / l and (m, l)
+        // blocks of 32 columns x 256 dims, [wave][dim half][dt % 8]..: the
         // layout prefill_kernel_w32d writes for its (pair, dim half) waves
-        const size_t blk = ((size_t)kh * a.n_qblocks + qb) * a.max_pieces + piece;
         const float inv_p = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-        half_t* po = a.part_o + blk * (NCOL * HD) + (size_t)wave * (32 * HD) + 8 * lane;
 #pragma unroll
-        for (int dt = 0; dt < 16; ++dt)
-#pragma unroll
-            for (int jp = 0; jp < 2; ++jp) store_part8<false>(po + (2 * dt + jp) * 512, oacc[dt], 8 * jp, inv_p);
-        if (h == 0) a.part_ml[blk * NCOL + c] = make_float2(m_use, l_tot);
+        for (int dt = 0; dt < 16; ++dt) store_part<false, HD, NCOL * HD>(a.part_o, P24, wu.slot, wave, dt, lane, oacc[dt], inv_p);
+        if (h == 0) a.part_ml[(size_t)wu.slot * NCOL + c] = make_float2(m_use, l_tot);
         return;
     }
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
@@ -1347,12 +1384,14 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32h(PrefillArgs a) {
 // M = max_p m_p, then srq and the output type. One workgroup per (query block, wave block of
 // 32 columns x 256 dims, kv head), laid out like the partials: thread (k, lane) owns the
 // lane's 8-dim runs k, k+4, .. (k < 4) of the 16 (dims tile, 4-row pair) runs, so every load
-// instruction reads a contiguous 1 KiB run. At most 8 pieces. HD 256: wave block w = columns 32w..; HD 512
+// instruction reads a contiguous 1 KiB run. At most 8 pieces, kMaxPieces24 with part24 (P24).
+// HD 256: wave block w = columns 32w..; HD 512
 // (prefill_kernel_w32d, NCOL 64, and prefill_kernel_w32h, NCOL 128): columns 32(w/2)..,
 // dims 256(w%2)..
-template <typename OUTT, int HD, int NCOL>
+template <typename OUTT, int HD, int NCOL, bool P24>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
-    constexpr int KT = HD == 256 ? 64 : 32, MAXP = 8;
+    constexpr int KT = HD == 256 ? 64 : 32, MAXP = P24 ? kMaxPieces24 : 8;
+    constexpr int NV = NCOL * HD, BLK = NV * (P24 ? 3 : 2);  // values and bytes of a piece's block
     const int qb = blockIdx.x, w = blockIdx.y, kh = blockIdx.z, tid = threadIdx.x;
     const int lane = tid & 63, k0 = tid >> 6;
     const int c = (HD == 256 ? 32 * w : 32 * (w >> 1)) + (lane & 31), h = lane >> 5;
@@ -1365,20 +1404,29 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     const int n_pieces = max(1, (n_tiles + a.split_tiles - 1) / a.split_tiles);
     const int s_idx = qb * BQ + c / G;
     if (n_pieces <= 1) return;
-    const size_t blk0 = ((size_t)kh * a.n_qblocks + qb) * a.max_pieces;
+    size_t blk0 = ((size_t)kh * a.n_qblocks + qb) * a.max_pieces;
+    if constexpr (P24) {  // slots in the work list's order: the pieces of the longer blocks come first
+        int before = 0;
+        for (int b = qb + 1 + lane; b < a.n_qblocks; b += 64) before += block_pieces(a, b, BQ, KT);
+        blk0 = (size_t)kh * a.pieces_per_head + __builtin_amdgcn_readlane(wave_prefix_sum(before), 63);
+    }
     // buffer ranges end at the block's last piece: the loads of absent pieces read zeros,
     // so all of them issue at once with no branch
     const rsrc_t rml = make_rsrc(a.part_ml + blk0 * NCOL, (uint32_t)n_pieces * NCOL * 8);
-    const rsrc_t ro = make_rsrc(a.part_o + blk0 * (NCOL * HD) + (size_t)w * (32 * 256), (uint32_t)n_pieces * NCOL * HD * 2);
+    const rsrc_t ro = make_rsrc(reinterpret_cast<const char*>(a.part_o) + blk0 * BLK, (uint32_t)(n_pieces * BLK));
     float2 ml[MAXP];
-    half8 ov[MAXP][4];
+    v4u32 ov[MAXP][4];
+    v2u32 ob[P24 ? MAXP : 1][4];
 #pragma unroll
     for (int p = 0; p < MAXP; ++p) ml[p] = bload_f32x2(rml, (p * NCOL + c) * 8);
 #pragma unroll
     for (int p = 0; p < MAXP; ++p)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)  // run k = k0 + 4i: dims tile k/2, 4-row pair k%2
-            ov[p][i] = bload_h8(ro, (p * NCOL * HD + (k0 + 4 * i) * 512 + 8 * lane) * 2);
+        for (int i = 0; i < 4; ++i) {  // run k = k0 + 4i: dims tile k/2, 4-row pair k%2
+            const int run = w * (32 * 256) + (k0 + 4 * i) * 512 + 8 * lane;
+            ov[p][i] = __builtin_amdgcn_raw_buffer_load_b128(ro, p * BLK + 2 * run, 0, 0);
+            if constexpr (P24) ob[p][i] = __builtin_amdgcn_raw_buffer_load_b64(ro, p * BLK + 2 * NV + run, 0, 0);
+        }
     float wt[MAXP];
     float M = kNegInf;
 #pragma unroll
@@ -1399,9 +1447,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int p = 0; p < MAXP; ++p) {
-            const half8 v = ov[p][i];
-            o[2 * i] += float4v{(float)v[0], (float)v[1], (float)v[2], (float)v[3]} * wt[p];
-            o[2 * i + 1] += float4v{(float)v[4], (float)v[5], (float)v[6], (float)v[7]} * wt[p];
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v[e] = P24 ? unpack24(ov[p][i], ob[P24 ? p : 0][i], e) : (float)__builtin_bit_cast(half8, ov[p][i])[e];
+            o[2 * i] += float4v{v[0], v[1], v[2], v[3]} * wt[p];
+            o[2 * i + 1] += float4v{v[4], v[5], v[6], v[7]} * wt[p];
         }
     if (s_idx >= a.S) return;
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
@@ -1418,43 +1469,51 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
 typedef void (*prefill_fn)(PrefillArgs);
 
 template <int HD, int G, bool HILO, bool KLO>
-static prefill_fn pick_w32_out(bool out32, bool split) {
+static prefill_fn pick_w32_out(bool out32, bool split, bool part24) {
     if constexpr (HD == 256) {
-        if (split) return out32 ? prefill_kernel_w32<G, float, HILO, KLO, true> : prefill_kernel_w32<G, half_t, HILO, KLO, true>;
-        return out32 ? prefill_kernel_w32<G, float, HILO, KLO, false> : prefill_kernel_w32<G, half_t, HILO, KLO, false>;
+        if (part24) return out32 ? prefill_kernel_w32<G, float, HILO, KLO, true, true> : prefill_kernel_w32<G, half_t, HILO, KLO, true, true>;
+        if (split) return out32 ? prefill_kernel_w32<G, float, HILO, KLO, true, false> : prefill_kernel_w32<G, half_t, HILO, KLO, true, false>;
+        return out32 ? prefill_kernel_w32<G, float, HILO, KLO, false, false> : prefill_kernel_w32<G, half_t, HILO, KLO, false, false>;
     } else {
         return out32 ? prefill_kernel_w32d<G, float, HILO, KLO> : prefill_kernel_w32d<G, half_t, HILO, KLO>;
     }
 }
 template <int HD, int G>
-static prefill_fn pick_w32(bool out32, bool hilo, bool klo, bool split) {
-    if (hilo) return klo ? pick_w32_out<HD, G, true, true>(out32, split) : pick_w32_out<HD, G, true, false>(out32, split);
-    return klo ? pick_w32_out<HD, G, false, true>(out32, split) : pick_w32_out<HD, G, false, false>(out32, split);
+static prefill_fn pick_w32(bool out32, bool hilo, bool klo, bool split, bool part24) {
+    if (hilo) return klo ? pick_w32_out<HD, G, true, true>(out32, split, part24) : pick_w32_out<HD, G, true, false>(out32, split, part24);
+    return klo ? pick_w32_out<HD, G, false, true>(out32, split, part24) : pick_w32_out<HD, G, false, false>(out32, split, part24);
 }
 template <int G>
-static prefill_fn pick_w32h(bool out32, bool qstage, bool ostage) {
-    if (qstage) return out32 ? prefill_kernel_w32h<G, float, true, true> : prefill_kernel_w32h<G, half_t, true, true>;
-    if (ostage) return out32 ? prefill_kernel_w32h<G, float, false, true> : prefill_kernel_w32h<G, half_t, false, true>;
-    return out32 ? prefill_kernel_w32h<G, float, false, false> : prefill_kernel_w32h<G, half_t, false, false>;
+static prefill_fn pick_w32h(bool out32, bool qstage, bool ostage, bool part24) {
+    if (part24) return out32 ? prefill_kernel_w32h<G, float, true, true, true> : prefill_kernel_w32h<G, half_t, true, true, true>;
+    if (qstage) return out32 ? prefill_kernel_w32h<G, float, true, true, false> : prefill_kernel_w32h<G, half_t, true, true, false>;
+    if (ostage) return out32 ? prefill_kernel_w32h<G, float, false, true, false> : prefill_kernel_w32h<G, half_t, false, true, false>;
+    return out32 ? prefill_kernel_w32h<G, float, false, false, false> : prefill_kernel_w32h<G, half_t, false, false, false>;
 }
-static prefill_fn pick_g_w32h(int G, bool out32, bool qstage, bool ostage) {
+static prefill_fn pick_g_w32h(int G, bool out32, bool qstage, bool ostage, bool part24) {
     switch (G) {
-        case 1: return pick_w32h<1>(out32, qstage, ostage);
-        case 2: return pick_w32h<2>(out32, qstage, ostage);
-        case 4: return pick_w32h<4>(out32, qstage, ostage);
-        case 8: return pick_w32h<8>(out32, qstage, ostage);
+        case 1: return pick_w32h<1>(out32, qstage, ostage, part24);
+        case 2: return pick_w32h<2>(out32, qstage, ostage, part24);
+        case 4: return pick_w32h<4>(out32, qstage, ostage, part24);
+        case 8: return pick_w32h<8>(out32, qstage, ostage, part24);
     }
     return nullptr;
 }
 template <int HD>
-static prefill_fn pick_g(int G, bool out32, bool hilo, bool klo, bool split) {
+static prefill_fn pick_g(int G, bool out32, bool hilo, bool klo, bool split, bool part24) {
     switch (G) {
-        case 1: return pick_w32<HD, 1>(out32, hilo, klo, split);
-        case 2: return pick_w32<HD, 2>(out32, hilo, klo, split);
-        case 4: return pick_w32<HD, 4>(out32, hilo, klo, split);
-        case 8: return pick_w32<HD, 8>(out32, hilo, klo, split);
+        case 1: return pick_w32<HD, 1>(out32, hilo, klo, split, part24);
+        case 2: return pick_w32<HD, 2>(out32, hilo, klo, split, part24);
+        case 4: return pick_w32<HD, 4>(out32, hilo, klo, split, part24);
+        case 8: return pick_w32<HD, 8>(out32, hilo, klo, split, part24);
     }
     return nullptr;
+}
+
+template <int HD, int NCOL>
+static prefill_fn pick_merge(bool out32, bool part24) {
+    if (part24) return out32 ? prefill_merge_kernel<float, HD, NCOL, true> : prefill_merge_kernel<half_t, HD, NCOL, true>;
+    return out32 ? prefill_merge_kernel<float, HD, NCOL, false> : prefill_merge_kernel<half_t, HD, NCOL, false>;
 }
 
 }  // namespace g4a
@@ -1462,16 +1521,17 @@ static prefill_fn pick_g(int G, bool out32, bool hilo, bool klo, bool split) {
 using namespace g4a;
 
 // Key split for short prompts: when the query blocks alone give fewer than 2 workgroups
-// per CU, long causal rows are cut into even pieces of at most split_tiles key tiles, the
-// longest block into 2 to 7 of them: as many as fill whole rounds of one piece a CU. Against
-// always about six pieces with the remainder in the last: hd 512 (f16 q, 1 KV head) S 1900
-// after 1100 187 -> 150 us a call, S 2047 108 -> 101, S 4096 321 -> 287; hd 256 (2 KV heads)
-// S 1500 40.3 -> 33.7, S 3000 82 -> 74; q and caches in f32, hd 256 S 1500 62 -> 53, hd 512
-// S 700 54 -> 43, S 2047 165 -> 148; relative rms error against f64 1.97e-4 -> 1.90e-4 (hd 256
-// S 1500), 2.91e-4 before and after (hd 512 S 1900). Where that rule already gave one round (hd 256 S 1024,
-// S 600 after 3000; hd 512 S 1024) the plan is the same.
+// per CU, long causal rows are cut into pieces of at most split_tiles key tiles. The longest block
+// takes about six with f16 partials, or, where that fills whole rounds of one piece a CU better,
+// 2 to 5 with 24-bit ones in the same workspace. A block's f16 partials round O to 2^-11, once a
+// piece, which averages out over six pieces but not over fewer: with f16 partials there too the
+// relative rms error against f64 of an f32 output grew by up to 31 % (hd 512, S 1900 after 1100, W 512:
+// 1.24e-4 -> 1.62e-4). In 24 bits it falls: 5.9e-5 there, 7.1e-5 instead of 1.41e-4 without the window.
+// us a call, six pieces -> this plan: hd 512 (f16 q, 1 KV head) S 1900 after 1100 192 -> 170, S 1280
+// 78 -> 60; hd 256 (2 KV heads) S 1500 43 -> 38, S 1000 after 1000 43 -> 36; q and caches in f32, hd
+// 256 S 1500 65 -> 57, hd 512 S 700 56 -> 47.
 struct PrefillSplit {
-    int split_tiles, max_pieces, n_qblocks, total_pieces;
+    int split_tiles, max_pieces, n_qblocks, total_pieces, part24;
     int kv_row0, kv_rows;  // f32 caches: the attended rows copied to f16
     // workspace layout [K16][V16][K16 low][q16][q16 low][partials][(m, l)]; base: the bytes
     // the unsplit call needs, total: with the split
@@ -1486,7 +1546,7 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // query columns a workgroup of the kernel that runs the call holds
 static int prefill_ncol(int HD, bool hilo) { return HD == 256 || !hilo ? 128 : 64; }
 static PrefillSplit prefill_split(const g4a_cfg* cfg, int S, int start_pos) {
-    PrefillSplit p{0, 1, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    PrefillSplit p{};
     const int HD = (int)cfg->head_dim;
     if ((HD != 256 && HD != 512) || S <= 0 || cfg->n_kv_heads == 0) return p;
     const int G = (int)(cfg->n_q_heads / cfg->n_kv_heads);
@@ -1530,29 +1590,33 @@ static PrefillSplit prefill_split(const g4a_cfg* cfg, int S, int start_pos) {
     const int room = (max_tiles + st - 1) / st;  // the workspace holds this many pieces a block
     if (room <= 1) return p;
     // of the piece counts that the workspace holds, the one whose rounds of 256 workgroups (one
-    // a CU) end first: a round lasts its longest piece, step us a tile and fixed us a piece.
-    // Measured, us a call (rounds x tiles): hd 512, S 1900 after 1100, 94-tile blocks: 3 x 16
-    // 180, 3 x 14 166, 2 x 24 175, 2 x 19 151, 1 x 47 164; S 2047, 64 tiles: 2 x 10 100, 2 x 16
-    // 128, 1 x 22 98; hd 256, S 3000, 2 KV heads, 47 tiles: 3 x 8 81, 2 x 12 74, 2 x 16 84
-    const float step = HD == 256 ? 1.5f : 3.0f, fixed = HD == 256 ? 7.0f : 5.0f;
-    int pieces = room;
-    float best = 0.0f;
-    for (int n = 2; n <= room; ++n) {
-        int tiles = (max_tiles + n - 1) / n, wgs = 0;
-        if (tiles < st_min) tiles = st_min;
+    // a CU) end first: a round lasts its longest piece, and a piece `fixed` tiles beyond its own.
+    // 24-bit partials take `wide` more beside the shorter f16-q tiles. Over 291 calls (both head
+    // sizes, q in f16 and at f32 accuracy, f16 and f32 caches, with and without a window, S 100 to
+    // 4000 after 0 to 4000) the choice is within 4.2 % of the best count, 0.1 % in the mean, and
+    // never slower than six f16 pieces.
+    const float fixed = HD == 256 ? 2.4f : 4.0f, wide = hilo ? 0.0f : 1.3f;
+    auto count = [&](int tiles) {  // the blocks' pieces (at most: a window's last block may have fewer)
+        int n = 0;
         for (int t = 0; t < max_tiles; t += tiles) {  // blocks of more than t tiles
             const int beyond = t * KT - start_pos;
-            if (W == 0 || t == 0 || t * KT < BQ + W - 1) wgs += p.n_qblocks - (beyond > 0 ? beyond / BQ : 0);
+            if (W == 0 || t == 0 || t * KT < BQ + W - 1) n += p.n_qblocks - (beyond > 0 ? beyond / BQ : 0);
         }
-        const float us = (float)((wgs * kvH + 255) / 256) * (tiles * step + fixed);
-        if (n == 2 || us < best) {
-            best = us;
+        return n;
+    };
+    auto cost = [&](int tiles, float extra) { return (float)((count(tiles) * kvH + 255) / 256) * (tiles + fixed + extra); };
+    float best = cost(st, 0.0f);
+    for (int n = 2; n <= kMaxPieces24 && n < room; ++n) {
+        const int tiles = std::max((max_tiles + n - 1) / n, st_min);
+        const float t = cost(tiles, wide);
+        if (t < best && 3 * count(tiles) <= 2 * room * p.n_qblocks) {
+            best = t;
             st = tiles;
-            pieces = (max_tiles + tiles - 1) / tiles;
+            p.part24 = 1;
         }
     }
     p.split_tiles = st;
-    p.max_pieces = pieces;
+    p.max_pieces = room;
     p.total_pieces = 0;
     for (int qb = 0; qb < p.n_qblocks; ++qb) {
         const int p0 = start_pos + qb * BQ;
@@ -1648,9 +1712,10 @@ extern "C" int g4a_prefill(const g4a_cfg* cfg, int S, int start_pos, const float
     // hd 512: prefill_kernel_w32h for f16 q (its 128 q registers a wave leave no room for
     // the low parts), prefill_kernel_w32d for G4A_Q_HILO
     const bool w32h = HD == 512 && !hilo;
-    const prefill_fn fn = HD == 256 ? pick_g<256>(G, out32, hilo, klo, split)
-                          : w32h    ? pick_g_w32h(G, out32, split, split || cfg->window > 0)
-                                    : pick_g<512>(G, out32, hilo, klo, split);
+    const bool part24 = split && sp.part24;
+    const prefill_fn fn = HD == 256 ? pick_g<256>(G, out32, hilo, klo, split, part24)
+                          : w32h    ? pick_g_w32h(G, out32, split, split || cfg->window > 0, part24)
+                                    : pick_g<512>(G, out32, hilo, klo, split, part24);
     if (!fn) {
         set_error("no prefill kernel for group size %d", G);
         return G4A_EUNSUPPORTED;
@@ -1681,6 +1746,7 @@ extern "C" int g4a_prefill(const g4a_cfg* cfg, int S, int start_pos, const float
     a.split_tiles = 0;
     a.max_pieces = 1;
     a.pieces_per_head = 0;
+    a.part24 = 0;
     a.part_o = nullptr;
     a.part_ml = nullptr;
     a.q16 = nullptr;
@@ -1721,7 +1787,8 @@ extern "C" int g4a_prefill(const g4a_cfg* cfg, int S, int start_pos, const float
         a.split_tiles = sp.split_tiles;
         a.max_pieces = sp.max_pieces;
         a.pieces_per_head = sp.total_pieces;
-        a.part_o = (half_t*)wsp;
+        a.part24 = part24;
+        a.part_o = wsp;
         a.part_ml = (float2*)(wsp + sp.o_bytes);
     }
     a.xcd_runs = a.split_tiles == 0 && cfg->window > 0;
@@ -1734,9 +1801,9 @@ extern "C" int g4a_prefill(const g4a_cfg* cfg, int S, int start_pos, const float
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_error(e, "prefill launch");
     if (a.split_tiles > 0) {
-        auto mf = HD == 256 ? (out32 ? prefill_merge_kernel<float, 256, 128> : prefill_merge_kernel<half_t, 256, 128>)
-                  : w32h    ? (out32 ? prefill_merge_kernel<float, 512, 128> : prefill_merge_kernel<half_t, 512, 128>)
-                            : (out32 ? prefill_merge_kernel<float, 512, 64> : prefill_merge_kernel<half_t, 512, 64>);
+        const prefill_fn mf = HD == 256 ? pick_merge<256, 128>(out32, part24)
+                              : w32h    ? pick_merge<512, 128>(out32, part24)
+                                        : pick_merge<512, 64>(out32, part24);
         // one workgroup per 32 columns x 256 dims of a query block
         hipLaunchKernelGGL(mf, dim3(a.n_qblocks, NCOL / 32 * (HD / 256), cfg->n_kv_heads), dim3(256), 0,
                            (hipStream_t)stream, a);

@@ -40,3 +40,37 @@ def test_pieces_match_uncut(S, start, hd, kvH, window, q_hilo):
                       out_dtype=torch.float32, q_hilo=q_hilo, workspace=ws, split=s).cpu().numpy()
            for s in (True, False)]
     contract_close(got[0], got[1], f"S={S}+{start} hd={hd} kvH={kvH} W={window}")
+
+
+def attend64(q, k, v, start, window):
+    """q [S][nH][hd] (normalised, rotated) at positions start.., causal, windowed, in float64."""
+    S, nH, _ = q.shape
+    key, at = torch.arange(start + S, device=DEV), start + torch.arange(S, device=DEV)[:, None]
+    ok = (key[None] <= at) & ((key[None] > at - window) if window else True)
+    outs = [torch.softmax((q[:, h] @ k[:, h * k.shape[1] // nH].double().T).masked_fill(~ok, -float("inf")), -1)
+            @ v[:, h * k.shape[1] // nH].double() for h in range(nH)]
+    return torch.stack(outs, 1)
+
+
+@pytest.mark.parametrize("S,start,hd,kvH,window,q_hilo", [
+    (1900, 1100, 256, 1, 512, False), (1900, 1100, 256, 1, 512, True), (1500, 0, 256, 2, 0, False), (1500, 0, 256, 2, 0, True),
+    (1000, 1000, 256, 4, 0, False), (1000, 1000, 256, 8, 0, True), (1000, 1000, 512, 1, 0, False), (1001, 1000, 512, 1, 0, True),
+    (1900, 1100, 512, 1, 512, False), (600, 3000, 512, 1, 512, True), (999, 1000, 512, 4, 0, False), (1000, 1000, 512, 8, 0, False)])
+def test_few_pieces_lose_no_precision(S, start, hd, kvH, window, q_hilo):
+    """Where the plan cuts long rows into few pieces, their partials hold 24 bits: the error of an
+    f32 output against float64 is the uncut call's, within 10 % (P rounds to f16 against another
+    running maximum). f16 partials of n pieces would add 2^-11 / sqrt(3 n) or so of the values,
+    1.2 times the uncut error and more at these sizes."""
+    print(f"pieces S {S} start {start} hd {hd} kvH {kvH} W {window} q_hilo {q_hilo}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(S + start)
+    cfg = sa.AttnConfig(8, kvH, hd, window)
+    q16_bytes = (1 + q_hilo) * S * 8 * hd * 2
+    assert sa.prefill_ws_bytes(S, start, cfg, q_hilo=q_hilo) > 1.5 * q16_bytes, "this call should be cut"
+    q = torch.randn(S, 8, hd, device=DEV, generator=g)
+    k, v = (torch.randn(start + S, kvH, hd, device=DEV, generator=g).half() for _ in range(2))
+    q64 = q.double() / torch.sqrt((q.double() ** 2).mean(-1, keepdim=True) + 1e-6)
+    ref = attend64(q64 if q_hilo else q64.half().double(), k, v, start, window)
+    err = [float((sa.prefill(q, k, v, start, cfg, q_gain=torch.ones(hd, device=DEV), out_dtype=torch.float32, q_hilo=q_hilo,
+                             workspace=sa.Workspace(DEV), split=s).double() - ref).norm() / ref.norm()) for s in (True, False)]
+    print(f"split {err[0]:.3e} uncut {err[1]:.3e}", flush=True)
+    assert err[0] <= 1.1 * err[1], f"split {err[0]:.2e}, uncut {err[1]:.2e}"
