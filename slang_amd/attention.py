@@ -283,9 +283,10 @@ def prefill(q, k_cache, v_cache, start_pos: int, cfg: AttnConfig, *, workspace: 
         q16 = (S * cfg.n_q_heads * cfg.head_dim * 2 + 255) // 256 * 256
         ws_bytes = 0 if cfg.head_dim == 256 else q16 * (2 if q_hilo else 1)
     ws = workspace.get(ws_bytes) if ws_bytes else None
+    # (the bytes asked for, not the buffer's: one grown by another call would let this one split)
     check(lib.g4a_prefill(ctypes.byref(c), S, int(start_pos), _ptr(q), _ptr(q_gain), _ptr(rope_cos),
                           _ptr(rope_sin), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(ws),
-                          0 if ws is None else ws.numel(), _stream()))
+                          ws_bytes, _stream()))
     return out
 
 

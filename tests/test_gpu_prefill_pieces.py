@@ -74,3 +74,17 @@ def test_few_pieces_lose_no_precision(S, start, hd, kvH, window, q_hilo):
                              workspace=sa.Workspace(DEV), split=s).double() - ref).norm() / ref.norm()) for s in (True, False)]
     print(f"split {err[0]:.3e} uncut {err[1]:.3e}", flush=True)
     assert err[0] <= 1.1 * err[1], f"split {err[0]:.2e}, uncut {err[1]:.2e}"
+
+
+def test_split_off_runs_uncut_on_a_grown_workspace():
+    """split=False after a call that grew the workspace to the split's size gives the uncut call's
+    values, bit for bit, not the split's."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    cfg = sa.AttnConfig(8, 1, 512)
+    q = torch.randn(600, 8, 512, device=DEV, generator=g)
+    k, v = (torch.randn(600, 1, 512, device=DEV, generator=g).half() for _ in range(2))
+    ws = sa.Workspace(DEV)
+    run = lambda w, s: sa.prefill(q, k, v, 0, cfg, q_gain=torch.ones(512, device=DEV), workspace=w, split=s)  # noqa: E731
+    cut, uncut = run(ws, True), run(sa.Workspace(DEV), False)
+    assert not torch.equal(cut, uncut)
+    assert torch.equal(run(ws, False), uncut)
