@@ -6,7 +6,7 @@
 //
 // MI355X design. At these shapes (K 1536 .. 12288, N 256 .. 24576) the products are bound by
 // how many bytes a CU moves per MFMA: a tile of BM tokens x BN outputs takes (BM + BN) * 128
-// bytes into LDS per 64-deep k-stage for BM * BN / 16 MFMA cycles, so the tile is as large as
+// bytes into LDS per 64-deep k-stage for BM * BN / 32 MFMA cycles, so the tile is as large as
 // the output allows, and the kernel keeps the loads away from the MFMAs:
 //  * k-stages come straight from HBM / L2 into LDS (buffer_load .. lds, 1 KiB per wave
 //    instruction, whole 128-byte row segments), ST stages deep. The DMAs are inline asm: as
@@ -24,10 +24,9 @@
 #include <stdio.h>
 #include <stdlib.h>
 
-#include <algorithm>
-
 #include "common.hpp"
 #include "gemm_offsets.hpp"
+#include "gemm_plan.hpp"
 
 namespace g4a {
 
@@ -397,76 +396,7 @@ using namespace g4a;
 
 namespace {
 
-constexpr int kCUs = 256;
-
-// The tiles a launch can take (tokens x weight rows), and what one costs in us as measured
-// with every CU busy: per 64-deep k-stage, and once for filling the pipeline and the epilogue.
-// A launch runs ceil(workgroups / 256) rounds (one workgroup a CU: the stages take 96 to 160
-// KiB of LDS), so the plan is the tile with the smallest rounds * (stages * step + fixed). At
-// K 1536, measured / estimated us: M 8000 N 12288 256x256 305 / 251, 256x192 329 / 269,
-// 128x128 385 / 367; M 1024 N 24576 256x192 83 / 67, 256x256 89 / 84; M 1900 N 3072 192x128
-// 24.4 / 21.3, 128x128 31 / 31, 256x256 38 / 42; M 1024 N 2560 128x128 15.0 / 15.3, 64x128
-// 21 / 22; M 300 N 2560 64x128 10.6 / 11.2, 128x128 13.7 / 15.3. `runs`: consecutive tiles on
-// one XCD (128x128 at M 2047 N 2048: 21.4 -> 19.4 us); the 256x256 tiles measured faster dealt
-// round-robin (M 2047 N 24576: 152 against 160 us).
-struct TileCfg {
-    int bm, bn;
-    float step, fixed;
-    int runs;
-};
-constexpr TileCfg kTiles[] = {{256, 256, 1.45f, 7.0f, 0}, {256, 192, 1.15f, 6.0f, 1}, {192, 128, 0.68f, 5.0f, 1},
-                              {128, 128, 0.45f, 4.5f, 1}, {64, 128, 0.30f, 4.0f, 1}};
-constexpr int kFirstSplit = 3;  // the tiles that have a split form
-// A split adds the tile's partials through memory: 0.25 us for each of a tile's and 0.03 us for
-// each workgroup of the launch, a fit to 64x128 and 128x128 splits of 2 to 8 at M 1 to 2047,
-// K 1536 to 12288 (the plan is within 5 % of the fastest tile and split of all 66 products; a
-// flat 3 + 0.8 us a split was up to 25 % off): N 256 K 1536 M 1 9.2 -> 7.6 us, M 1024 10.3 ->
-// 9.6; N 1536 K 2048 M 300 14.0 -> 11.5.
-constexpr float kMergeEach = 0.25f, kMergeGroup = 0.03f;
-
-// The workspace contract (g4a_gemm16_ws_bytes): launches of fewer 128 x 64 output tiles than
-// CUs may split k up to `max_splits` times, at least four k-stages each, and are asked for that
-// many f32 copies of their (padded) output behind the ticket words. The plan below splits
-// fewer times or not at all where that is faster, and never needs more.
-constexpr int kSplitBelow = 256, kSplitTarget = 768, kSplitMinSteps = 4;
-constexpr size_t kTicketBytes = G4A_GEMM_TICKET_BYTES;
-static_assert(kSplitBelow * 4 <= kTicketBytes, "a ticket word per split tile");
-
-struct SplitRoom {
-    int max_splits;
-    size_t ws_bytes;  // tickets + partials, 0 without a split
-};
-SplitRoom split_room(int M, int K, int n_mats, const g4a_gemm_mat* mats) {
-    long tiles = 0;
-    for (int i = 0; i < n_mats; ++i) tiles += (long)(mats[i].n / 64) * ((M + 127) / 128);
-    SplitRoom r{1, 0};
-    if (tiles < kSplitBelow) r.max_splits = (int)std::max(1l, std::min((long)K / 64 / kSplitMinSteps, kSplitTarget / tiles));
-    if (r.max_splits > 1) r.ws_bytes = kTicketBytes + (size_t)tiles * r.max_splits * 128 * 64 * 4;
-    return r;
-}
-
-struct GemmPlan {
-    int cfg, tiles, splits;
-};
-// rows: weight rows of each matrix (2 n for the gate/up pair, whose tiles hold rows of both)
-GemmPlan gemm_plan(int M, int K, int n_mats, const int* rows, int max_splits) {
-    GemmPlan best{0, 0, 1};
-    float least = 0;
-    for (int c = 0; c < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++c) {
-        const TileCfg& t = kTiles[c];
-        long tiles = 0;
-        for (int i = 0; i < n_mats; ++i) tiles += (long)((rows[i] + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm);
-        for (int s = 1; s <= (c >= kFirstSplit && tiles <= (long)(kTicketBytes / 4) ? max_splits : 1); ++s) {
-            const long rounds = (tiles * s + kCUs - 1) / kCUs;
-            const float cost = rounds * ((K / 64 + s - 1) / s * t.step + t.fixed) + (s > 1 ? kMergeEach * s + kMergeGroup * (tiles * s) : 0.0f);
-            if (!best.tiles || cost < least) {
-                best = {c, (int)tiles, s};
-                least = cost;
-            }
-        }
-    }
-    return best;
-}
+static_assert(kGemmTicketBytes == G4A_GEMM_TICKET_BYTES, "the header's ticket words");
 
 int gemm_check(int M, int K, const void* a_f16, int n_mats, const g4a_gemm_mat* mats) {
     if (M <= 0 || K <= 0 || K % 64) {
@@ -500,16 +430,20 @@ void gemm_launch(const GemmPlan& pl, const Gemm16Args& g, hipStream_t s) {
         if (pl.cfg == 0) hipLaunchKernelGGL((gemm16_kernel<256, 256, 2, 4, 2, 2, MODE>), grid, dim3(512), 0, s, g);
         if (pl.cfg == 1) hipLaunchKernelGGL((gemm16_kernel<256, 192, 2, 2, 2, 1, MODE>), grid, dim3(256), 0, s, g);
         if (pl.cfg == 2) hipLaunchKernelGGL((gemm16_kernel<192, 128, 2, 2, 4, 1, MODE>), grid, dim3(256), 0, s, g);
+        if (pl.cfg == 3) hipLaunchKernelGGL((gemm16_kernel<128, 128, 2, 2, 2, 2, MODE>), grid, dim3(256), 0, s, g);
     }
-    if (pl.cfg == 3) hipLaunchKernelGGL((gemm16_kernel<128, 128, 2, 2, 4, 1, MODE>), grid, dim3(256), 0, s, g);
-    if (pl.cfg == 4) hipLaunchKernelGGL((gemm16_kernel<64, 128, 2, 4, 6, 2, MODE>), grid, dim3(512), 0, s, g);
+    if (pl.cfg == 4) hipLaunchKernelGGL((gemm16_kernel<128, 128, 2, 2, 4, 1, MODE>), grid, dim3(256), 0, s, g);
+    if (pl.cfg == 5) hipLaunchKernelGGL((gemm16_kernel<64, 128, 2, 4, 6, 2, MODE>), grid, dim3(512), 0, s, g);
+    if (pl.cfg == 6) hipLaunchKernelGGL((gemm16_kernel<64, 128, 2, 4, 3, 4, MODE>), grid, dim3(512), 0, s, g);
 }
 
 int gemm_run(int M, int K, const void* a_f16, int n_mats, const g4a_gemm_mat* mats, void* ws, size_t ws_bytes,
              void* stream) {
     const int rc = gemm_check(M, K, a_f16, n_mats, mats);
     if (rc != G4A_OK) return rc;
-    const SplitRoom room = split_room(M, K, n_mats, mats);
+    int rows[3];
+    for (int i = 0; i < n_mats; ++i) rows[i] = mats[i].n;
+    const SplitRoom room = split_room(M, K, n_mats, rows);
     if (ws && ws_bytes < room.ws_bytes) {
         set_error("workspace of %zu bytes, this product needs %zu (g4a_gemm16_ws_bytes)", ws_bytes, room.ws_bytes);
         return G4A_EWORKSPACE;
@@ -518,8 +452,6 @@ int gemm_run(int M, int K, const void* a_f16, int n_mats, const g4a_gemm_mat* ma
         set_error("the workspace must be 256-byte aligned");
         return G4A_EINVAL;
     }
-    int rows[3];
-    for (int i = 0; i < n_mats; ++i) rows[i] = mats[i].n;
     const GemmPlan pl = gemm_plan(M, K, n_mats, rows, ws ? room.max_splits : 1);
     const TileCfg& tc = kTiles[pl.cfg];
     Gemm16Args g = {};
@@ -544,7 +476,7 @@ int gemm_run(int M, int K, const void* a_f16, int n_mats, const g4a_gemm_mat* ma
     g.splits = pl.splits;
     if (pl.splits > 1) {
         g.ticket = reinterpret_cast<unsigned*>(ws);
-        g.part = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + kTicketBytes);
+        g.part = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + kGemmTicketBytes);
         gemm_launch<kSplitK>(pl, g, (hipStream_t)stream);
     } else {
         gemm_launch<kPlain>(pl, g, (hipStream_t)stream);
@@ -605,9 +537,12 @@ extern "C" int g4a_gemm16_geglu(int M, int K, const void* a_f16, const void* w_g
 
 extern "C" size_t g4a_gemm16_ws_bytes(int M, int K, int n_mats, const g4a_gemm_mat* mats) {
     if (M <= 0 || K <= 0 || K % 64 || n_mats < 1 || n_mats > 3 || !mats) return 0;
-    for (int i = 0; i < n_mats; ++i)
+    int rows[3];
+    for (int i = 0; i < n_mats; ++i) {
         if (mats[i].n <= 0 || mats[i].n % 128) return 0;
-    return split_room(M, K, n_mats, mats).ws_bytes;
+        rows[i] = mats[i].n;
+    }
+    return split_room(M, K, n_mats, rows).ws_bytes;
 }
 
 extern "C" int g4a_gemm16_ws(int M, int K, const void* a_f16, int n_mats, const g4a_gemm_mat* mats, void* ws,

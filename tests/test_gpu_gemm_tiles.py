@@ -34,11 +34,19 @@ def close(got, a, w, what):
     assert not bad.any(), f"{what}: {int(bad.sum())} of {bad.numel()} products off"
 
 
-# the tile that the plan takes, by its measured costs: 256 x 256, 256 x 192, 192 x 128,
-# 128 x 128, 64 x 128
+# Which tile a shape runs on is the plan's choice: test_gemm_plan.py holds that these lists reach
+# all of them, each with a ragged last tile.
 SHAPES = [(2047, 64, (24576,)), (2040, 192, (12288, 12160)), (1000, 128, (24448,)), (2047, 128, (4096, 512, 512)),
           (1893, 192, (3072,)), (1893, 64, (2048, 384, 640)), (1024, 320, (2048, 512)), (513, 64, (4096,)),
-          (1, 64, (128,)), (65, 448, (384, 128)), (63, 128, (24576,))]
+          (1, 64, (128,)), (65, 448, (384, 128)), (63, 128, (24576,)),
+          (1893, 320, (12288, 12160)), (4000, 320, (4096,)), (1893, 512, (4096, 512, 512)), (1893, 640, (2048, 512)),
+          (1500, 640, (2048, 384, 640)), (513, 1536, (4096,)), (700, 1536, (2048, 384, 640)), (65, 2048, (384, 128)),
+          (1, 2048, (128,)), (1, 128, (128,))]
+SPLIT_SHAPES = [(77, 4096, (128, 384)), (1, 8192, (128,)), (1000, 12288, (1536,)), (130, 6144, (1536,)), (40, 1024, (128,)),
+                (200, 1344, (256,)), (300, 2048, (1536,)), (1, 1536, (256,)), (700, 6144, (1536,)),
+                (200, 16384, (2048, 256, 256)), (77, 16384, (384, 128)), (65, 12288, (1536,))]
+GEGLU_SHAPES = [(2047, 64, 12288), (1000, 128, 12224), (1893, 192, 1536), (1024, 320, 1216), (65, 64, 64),
+                (1893, 320, 12224), (300, 1088, 12224), (1893, 640, 1216), (1000, 1536, 1216), (65, 2048, 64), (65, 448, 64)]
 
 
 @pytest.mark.parametrize("M,K,ns", SHAPES)
@@ -57,8 +65,7 @@ def test_every_tile_matches_float64(M, K, ns):
     assert torch.equal(q[:M], want) and (q[M:] == 7.0).all()
 
 
-@pytest.mark.parametrize("M,K,ns", [(77, 4096, (128, 384)), (1, 8192, (128,)), (1000, 12288, (1536,)), (130, 6144, (1536,)),
-                                    (40, 1024, (128,)), (200, 1344, (256,)), (300, 2048, (1536,)), (1, 1536, (256,))])
+@pytest.mark.parametrize("M,K,ns", SPLIT_SHAPES)
 def test_split_tiles_match_float64_and_repeat(M, K, ns):
     print(f"gemm16 split M {M} K {K} n {ns}", flush=True)
     a, ws = operands(M, K, ns, M + K)
@@ -96,7 +103,7 @@ def geglu_pair(a, wg, wu, gq, uq, oq, lut):
     return out[:M], geglu16(g, u, gq, uq, oq, gelu_lut=lut)
 
 
-@pytest.mark.parametrize("M,K,n", [(2047, 64, 12288), (1000, 128, 12224), (1893, 192, 1536), (1024, 320, 1216), (65, 64, 64)])
+@pytest.mark.parametrize("M,K,n", GEGLU_SHAPES)
 @pytest.mark.parametrize("table", [True, False])
 def test_geglu_tiles_equal_the_divided_form(M, K, n, table):
     print(f"gemm16_geglu M {M} K {K} n {n} table {table}", flush=True)
