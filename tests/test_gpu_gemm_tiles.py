@@ -73,8 +73,9 @@ def test_split_tiles_match_float64_and_repeat(M, K, ns):
     mats = [(w, o[:M], None) for w, o in zip(ws, outs)]
     gws = sa.GemmWorkspace()
     gws.get(sa.gemm16_ws_bytes(M, K, ns))
-    gws.buf[sa._lib.GEMM_TICKET_BYTES:].fill_(0xFF)  # stale partials are NaN and must not be read
+    parts = gws.buf[sa._lib.GEMM_TICKET_BYTES:].fill_(0xFF)  # stale partials are NaN and must not be read
     sa.gemm16(a, mats, gws)
+    assert (parts != 0xFF).any(), "this product should split K"
     first = [o.clone() for o in outs]
     sa.gemm16(a, mats, gws)
     for i, (w, o, f) in enumerate(zip(ws, outs, first)):

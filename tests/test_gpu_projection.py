@@ -255,11 +255,23 @@ def test_prefill_qkv_block():
     srq_close(q.cpu().numpy(), refq.astype(np.float32), 0.03125, "q")
 
 
-@pytest.mark.parametrize("M,K,ns", [(1024, 6144, (1536,)), (1024, 2048, (1536,)), (1024, 1536, (256,)),
-                                    (200, 1536, (256,)), (512, 1536, (2048, 256, 256)), (77, 4096, (128, 384))])
-def test_gemm16_split_k_matches_oracle(M, K, ns):
+def stale_partials(gws, nbytes):
+    """Grow gws to nbytes, tickets zero and every partial NaN; returns a check that a call stored
+    partials there, the proof that it split K (the workspace's size only says that it may)."""
+    gws.get(nbytes)
+    parts = gws.buf[sa._lib.GEMM_TICKET_BYTES:]
+    parts.fill_(0xFF)
+    return lambda: bool((parts != 0xFF).any())
+
+
+@pytest.mark.parametrize("M,K,ns,splits", [(1024, 6144, (1536,), True), (1024, 2048, (1536,), False),
+                                           (1024, 1536, (256,), True), (200, 1536, (256,), True),
+                                           (512, 1536, (2048, 256, 256), False), (77, 4096, (128, 384), True),
+                                           (300, 2048, (1536,), True), (128, 4096, (2048, 256, 256), True)])
+def test_gemm16_split_k_matches_oracle(M, K, ns, splits):
     """g4a_gemm16_ws: launches with few output tiles split K over several workgroups per tile
-    and add the f32 partials in split order. The outputs meet the same bounds as the unsplit
+    and add the f32 partials in split order (`splits`: where the plan takes that, rather than the
+    unsplit launch that the same workspace allows). The outputs meet the same bounds as the unsplit
     GEMM, a repeat call is bit-identical (the sum order does not depend on which workgroup
     finishes last), rows past M are not stored, and the tickets are left at zero."""
     rng = np.random.default_rng(M + K + 7 * len(ns))
@@ -276,8 +288,10 @@ def test_gemm16_split_k_matches_oracle(M, K, ns):
     gws = sa.GemmWorkspace()
     _, _, tab = sa.projection._gemm_table(a16, mats)
     need = sa._lib.load().g4a_gemm16_ws_bytes(M, K, len(ns), tab)
-    assert need > 0, "this shape should split K"
+    assert need > 0, "this shape may split K"
+    stored = stale_partials(gws, need)
     sa.gemm16(a16, mats, gws)
+    assert stored() == splits, "split K" if not splits else "did not split K"
     first = [o.clone() for o in outs]
     sa.gemm16(a16, mats, gws)
     torch.cuda.synchronize()
@@ -365,8 +379,10 @@ def test_split_gemm_and_geglu_gemm_replay_in_a_graph():
         sa.gemm16(a16, [(w, o1, None, 0.5)], gws)
         sa.gemm16_geglu(b16, wg, wu, 0.05, 0.04, 0.05, out=o2)
 
+    stored = stale_partials(gws, sa.gemm16_ws_bytes(M, K, (n,)))
     run()
     torch.cuda.synchronize()
+    assert stored(), "the GEMM of this test should split K"
     ref1, ref2 = o1.clone(), o2.clone()
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
@@ -379,9 +395,11 @@ def test_split_gemm_and_geglu_gemm_replay_in_a_graph():
     for rep in range(3):
         o1.fill_(float("nan"))
         o2.fill_(float("nan"))
+        stored = stale_partials(gws, 0)
         torch.cuda.synchronize()
         g.replay()
         torch.cuda.synchronize()
+        assert stored(), f"replay {rep}: no partials stored"
         assert torch.equal(o1, ref1), f"replay {rep}: split GEMM differs"
         assert torch.equal(o2, ref2), f"replay {rep}: gate/up GEMM differs"
         assert not gws.buf[:sa._lib.GEMM_TICKET_BYTES].any(), "tickets left non-zero"
@@ -394,7 +412,8 @@ def test_split_gemm_workspace_shared_across_shapes():
     the tickets are zero after each call."""
     rng = np.random.default_rng(9)
     shared = sa.GemmWorkspace()
-    for M, K, n in [(1024, 2048, 1536), (1024, 1536, 256), (512, 6144, 1536), (1024, 2048, 1536), (200, 1536, 256)]:
+    for M, K, n in [(1024, 2048, 1536), (1024, 1536, 256), (512, 6144, 1536), (700, 6144, 1536), (1024, 2048, 1536),
+                    (300, 2048, 1536), (200, 1536, 256)]:
         a16 = sa.srqh(t(rng.standard_normal((M, K)).astype(np.float32)), 0.0625)
         w = sa.dequant(dev_words(words(rng, n * K // 8)), t(rng.random(n).astype(np.float32) * 0.01 + 0.02), K, n)
         o1 = torch.empty(M, n, device=DEV, dtype=torch.float16)
