@@ -25,6 +25,14 @@ def operands(M, K, ns, seed):
     return a, [(0.05 * torch.randn(n, K, device=DEV, generator=g)).half() for n in ns]
 
 
+def srq_of_f16(step):
+    """[65536] f32: srq(f32(v), step) of the f16 v of each bit pattern, by an IEEE f32 division."""
+    v = np.arange(65536, dtype=np.uint16).view(np.float16).astype(np.float32)
+    s = np.float32(step)
+    with np.errstate(all="ignore"):
+        return torch.from_numpy(np.clip(np.rint(v / s), -128, 127).astype(np.float32) * s if step else v).to(DEV)
+
+
 def close(got, a, w, what):
     ref = a.double() @ w.double().T
     mag = a.double().abs() @ w.double().abs().T
@@ -58,11 +66,26 @@ def test_every_tile_matches_float64(M, K, ns):
     for i, (w, o) in enumerate(zip(ws, outs)):
         close(o[:M], a, w, f"matrix {i}")
         assert (o[M:] == 7.0).all(), "stores past M"
-    # the q path: srq of the same f16 products, exactly
+    # the q path: srq of the same f16 products, exactly, at a power of two, steps that have f16 values
+    # at their ties, and outside the range that the refined products take (0, 1e-14)
     q = torch.full((M + 2, ns[0]), 7.0, device=DEV)
-    sa.gemm16(a, [(ws[0], q[:M], 0.03125)])
-    want = torch.clamp(torch.round(outs[0][:M].float() / 0.03125), -128, 127) * 0.03125
-    assert torch.equal(q[:M], want) and (q[M:] == 7.0).all()
+    bits = outs[0][:M].view(torch.int16).int() & 0xFFFF
+    for step in (0.03125, 7 / 256, 13 / 1024, 0.0, 1e-14):
+        sa.gemm16(a, [(ws[0], q[:M], step)])
+        assert torch.equal(q[:M], srq_of_f16(step)[bits]), f"step {step}"
+        assert (q[M:] == 7.0).all(), "stores past M"
+
+
+@pytest.mark.parametrize("step", [7 / 256, 13 / 1024, 41 / 2048, 0.0137, 0.3330001, 1e-6, 1e-14, 1e14, 0.0])
+def test_q_path_of_every_f16_value(step):
+    """Every finite f16 value as a product of the q path. The first steps put f16 values at ties that
+    x (1 / step), rounded, takes to the wrong side 78, 22 and 8 times."""
+    print(f"q path every f16 step {step}", flush=True)
+    v = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    v = torch.where(torch.isfinite(v), v, torch.zeros(())).half().to(DEV)
+    q = torch.empty(64, 1024, device=DEV)
+    sa.gemm16(torch.eye(64, device=DEV).half(), [(v.view(1024, 64), q, step)])
+    assert torch.equal(q.T, srq_of_f16(step)[v.view(torch.int16).int() & 0xFFFF].view(1024, 64))
 
 
 @pytest.mark.parametrize("M,K,ns", SPLIT_SHAPES)
