@@ -16,7 +16,9 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("S,start,hd,kvH,window,q_hilo", [
-    (97, 0, 256, 2, 0, False),  # 2 tiles: the longest block alone is cut
+    (160, 0, 256, 2, 0, False),  # 3 tiles: the last block alone is cut, 2 tiles and 1
+    (97, 0, 512, 1, 0, False),  # 4 tiles are one piece: not cut, as the next
+    (97, 0, 256, 2, 0, False),
     (97, 160, 512, 1, 0, False),
     (300, 0, 512, 1, 0, False),
     (1500, 0, 256, 2, 0, False),  # one round of 4 pieces a block
@@ -35,6 +37,9 @@ def test_pieces_match_uncut(S, start, hd, kvH, window, q_hilo):
     k, v = (torch.randn(start + S, kvH, hd, generator=g).to(DEV).half() for _ in range(2))
     k *= hd ** -0.5  # scores of order 1: every key counts
     cos, sin = (torch.as_tensor(x).to(DEV) for x in sa.rope_tables(np.arange(start, start + S), hd, 1e6))
+    uncut_bytes = 0 if hd == 256 else -(-S * 8 * hd * 2 // 256) * 256 * (1 + q_hilo)  # q in f16
+    cut = sa.prefill_ws_bytes(S, start, cfg, q_hilo=q_hilo) > uncut_bytes
+    assert cut == (start + S > 97), "this call should be cut" if not cut else "this call should not be cut"
     ws = sa.Workspace(DEV)
     got = [sa.prefill(q, k, v, start, cfg, q_gain=torch.ones(hd, device=DEV), rope_cos=cos, rope_sin=sin,
                       out_dtype=torch.float32, q_hilo=q_hilo, workspace=ws, split=s).cpu().numpy()
