@@ -45,7 +45,7 @@ struct PrefillArgs {
     // key split of long causal rows: split_tiles = 0 means none;
     // otherwise a workgroup covers at most split_tiles key tiles of its query block and
     // blocks with more tiles leave partials for prefill_merge_kernel (part24: in 24 bits a value)
-    int split_tiles, max_pieces, pieces_per_head, part24;
+    int split_tiles, max_pieces, pieces_per_head;
     int xcd_runs;  // prefill_kernel_w32 unsplit: 1-D grid, query blocks in contiguous runs per XCD
     int xcd_heads;  // unsplit causal: 1-D grid, kv head h on XCDs 8h/kvH .., its blocks longest first
     const half_t* q16;  // prefill_kernel_w32: q already prepared in f16 (qprep_kernel), or NULL
@@ -59,6 +59,7 @@ struct PrefillArgs {
     // list's order: with short blocks' absent pieces left out, more of these larger blocks fit.
     void* part_o;
     float2* part_ml;
+    int part24;  // last, where the kernels without it do not load it
 };
 
 constexpr int kMaxPieces24 = 5;  // pieces of a block with part24
@@ -721,10 +722,11 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32(PrefillArgs a) {
     // ---- epilogue: column sum over both halves, normalise, srq, store 4 dims at a time
     const float l_tot = add32(l_run);
     if (SPLITK && n_pieces > 1) {  // a piece of a split query block: O / l and (m, l)
+        const int slot = P24 ? wu.slot : (kh * a.n_qblocks + qb) * a.max_pieces + piece;
         const float inv_p = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) store_part<true, HD, NCOL * HD>(a.part_o, P24, wu.slot, wave, dt, lane, oacc[dt], inv_p);
-        if (h == 0) a.part_ml[(size_t)wu.slot * NCOL + c] = make_float2(m_use, l_tot);
+        for (int dt = 0; dt < 8; ++dt) store_part<true, HD, NCOL * HD>(a.part_o, P24, slot, wave, dt, lane, oacc[dt], inv_p);
+        if (h == 0) a.part_ml[(size_t)slot * NCOL + c] = make_float2(m_use, l_tot);
         return;
     }
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
@@ -1332,13 +1334,17 @@ __global__ __launch_bounds__(256) void prefill_kernel_w32h(PrefillArgs a) {
                    "+a"(oacc[6]), "+a"(oacc[7]), "+a"(oacc[8]), "+a"(oacc[9]), "+a"(oacc[10]), "+a"(oacc[11]),
                    "+a"(oacc[12]), "+a"(oacc[13]), "+a"(oacc[14]), "+a"(oacc[15]));
     const float l_tot = add32(l_run);
-    if (QSTAGE && n_pieces > 1) {  // a piece of a split query block: O / l and (m, l)
+    if (n_pieces > 1) {  // a piece of a split query block: O / l and (m, l)
         // blocks of 32 columns x 256 dims, [wave][dim half][dt % 8]..: the
-        // layout prefill_kernel_w32d writes for its (pair, dim half) waves
+        // layout prefill_kernel_w32d writes for its (pair, dim half) waves. The launches without
+        // a split never come here, but are slower without this code (the registers fall otherwise):
+        // S 8192 global 796 -> 814 us a call, 1 KV head. So are those with f16 partials if their slot is
+        // held over the loop (S 600 after 3000 86 -> 90).
+        const int slot = P24 ? wu.slot : (kh * a.n_qblocks + qb) * a.max_pieces + piece;
         const float inv_p = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
 #pragma unroll
-        for (int dt = 0; dt < 16; ++dt) store_part<false, HD, NCOL * HD>(a.part_o, P24, wu.slot, wave, dt, lane, oacc[dt], inv_p);
-        if (h == 0) a.part_ml[(size_t)wu.slot * NCOL + c] = make_float2(m_use, l_tot);
+        for (int dt = 0; dt < 16; ++dt) store_part<false, HD, NCOL * HD>(a.part_o, P24, slot, wave, dt, lane, oacc[dt], inv_p);
+        if (h == 0) a.part_ml[(size_t)slot * NCOL + c] = make_float2(m_use, l_tot);
         return;
     }
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
