@@ -1533,7 +1533,7 @@ using namespace g4a;
 // piece, which averages out over six pieces but not over fewer: with f16 partials there too the
 // relative rms error against f64 of an f32 output grew by up to 31 % (hd 512, S 1900 after 1100, W 512:
 // 1.24e-4 -> 1.62e-4). In 24 bits it falls: 5.9e-5 there, 7.1e-5 instead of 1.41e-4 without the window.
-// us a call, six pieces -> this plan: hd 512 (f16 q, 1 KV head) S 1900 after 1100 192 -> 170, S 1280
+// us a call, six pieces -> this plan: hd 512 (f16 q, 1 KV head) S 1900 after 1100 192 -> 161, S 1280
 // 78 -> 60; hd 256 (2 KV heads) S 1500 43 -> 38, S 1000 after 1000 43 -> 36; q and caches in f32, hd
 // 256 S 1500 65 -> 57, hd 512 S 700 56 -> 47.
 struct PrefillSplit {

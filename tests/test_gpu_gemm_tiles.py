@@ -1,7 +1,7 @@
 """g4a_gemm16 / g4a_gemm16_ws / g4a_gemm16_geglu at the edges of every output tile the launch
-plan can take (csrc/gemm.hip kTiles): ragged tokens and outputs, one k-stage, fewer stages than
+plan can take (csrc/gemm_plan.hpp kTiles): ragged tokens and outputs, one k-stage, fewer stages than
 the pipeline holds, grouped matrices whose last tiles are partly empty, and a split with the
-smallest tile. Products against float64 (on the GPU, the operands being f16 exactly):
+smallest tiles. Products against float64 (on the GPU, the operands being f16 exactly):
 
     |got - f16(ref)| <= one f16 ulp of ref + K 2^-24 sum|a w|
 
